@@ -18,6 +18,7 @@ struct KrylovScalars {
     double tol, tol2, delta2, breakdown;
     long long iter, nit, maxit;
     int done, flag;
+    int stuck;         // a wait of the resident kernel ran out (resident.h)
     double scaled[2];  // scaled residual: max|A x - b|, max|diag * x|
 };
 
@@ -120,7 +121,7 @@ void launch_flush(const Launch& L, int n, double* x64, float* x32);
 // entry differs from its mirrored upper entry (ref_blocks(n) doubles).
 void launch_dia_symcheck(const Launch& L, const KView<double>& kv, const double* vals, double* part,
                          size_t part_cap);
-// ks->done = 0 and / or ks->iter = 0 (on the stream, before a seed).
+// ks->done = ks->stuck = 0 and / or ks->iter = 0 (on the stream, before a seed).
 void launch_reset_events(const Launch& L, KrylovScalars* ks, bool clear_done, bool clear_iter);
 template <typename T>
 void launch_convert(const Launch& L, int64_t n, const double* src, T* dst);

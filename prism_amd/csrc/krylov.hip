@@ -11,7 +11,8 @@
 //      x += alpha M^-1 p + omega M^-1 s; r' = s - omega t; p' = r' + beta (p - omega v);
 //      partials of (rhat, p'), (r', r')                                       (stream)
 // Three reductions, the fewest BiCGSTAB admits, each taken at a kernel boundary that the
-// SpMVs need anyway.  After a seed (start, restart, reliable update) an entry kernel forms p
+// SpMVs need anyway.  Systems whose rows fit the registers of the device run these iterations
+// inside one kernel instead (resident.hip).  After a seed (start, restart, reliable update) an entry kernel forms p
 // from the seeded r.  The five-kernel form (p and s updates in kernels of their own, (r0, v)
 // reduced directly) is selectable for comparison.
 // Each SpMV gathers a single vector (one L2 line per neighbour).  V, which writes no partial
@@ -1326,7 +1327,7 @@ __global__ void __launch_bounds__(BS) k_seed(KView<T> kv, const double* r64, int
 // Clears the event state before a seed: done (clear_done) and the iteration counter (clear_iter).
 __global__ void k_reset_events(KrylovScalars* ks, int clear_done, int clear_iter) {
     if (threadIdx.x == 0) {
-        if (clear_done) ks->done = 0;
+        if (clear_done) ks->done = ks->stuck = 0;
         if (clear_iter) ks->iter = 0;
     }
 }

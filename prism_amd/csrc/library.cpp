@@ -9,6 +9,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 #include <chrono>
 #include <cmath>
@@ -26,6 +27,7 @@
 #include "internal.h"
 #include "krylov.h"
 #include "output.h"
+#include "resident.h"
 #include "sgs.h"
 
 using namespace prism_hip;
@@ -124,6 +126,7 @@ struct prism_ctx {
     std::vector<std::string> order;
     KrylovScalars* hks{nullptr};  // pinned mirror
     unsigned char* scratch{nullptr};  // this device's static scratch array (scratch_address)
+    int n_cu{0};                      // compute units of the device
 
     Launch launch() {
         Launch L;
@@ -204,11 +207,18 @@ struct prism_mesh {
     DevBuf<int32_t> v2c_off, v2c_sbase, v2c_cell;
     DevBuf<double> idw;
     DevBuf<double> pts;  // point values of the last export (grows to the widest field exported)
+    int wmax{0};         // entries of the widest sliced-ELL slice
     DMesh dm{};
     SgsCache sgs;
 };
 
 namespace {
+
+int widestSlice(const std::vector<int32_t>& sell_off) {
+    int32_t w = 0;
+    for (size_t s = 0; s + 1 < sell_off.size(); ++s) w = std::max(w, sell_off[s + 1] - sell_off[s]);
+    return (int)(w >> 6);
+}
 
 int8_t kindCode(const std::string& k) {
     if (k == "fixed") return BC_FIXED;
@@ -462,6 +472,10 @@ struct Workspace {  // Krylov buffers of one equation, allocated on first solve
     DevBuf<KrylovScalars> ks;
     DevBuf<double> aval, bt, part_ref;  // reference-cell deflation: matrix, rhs, partials
     DevBuf<double> xsave;                // FP32 refinement: x at the best reliable update so far
+    DevBuf<double> d_pub;                // resident kernel: exchange buffers and partial sums
+    DevBuf<float> f_pub;
+    DevBuf<unsigned long long> slots;
+    bool scratch{false};                 // bound to the static scratch array (bindScratch)
     // multicolour SGS-preconditioned iteration (position numbering)
     struct Sgs {
         DevBuf<double> sval, d, dinv, x, b, r, r0, p, v, y, s, z, t, e, part_x, part_v, part_t;
@@ -486,6 +500,7 @@ struct Workspace {  // Krylov buffers of one equation, allocated on first solve
     // sliced ELL) may use to slices of [base, base + bytes) instead of device allocations
     // (the allocation-free entry point).  Fails with PRISM_ERR_INVALID when they do not fit.
     void bindScratch(unsigned char* base, size_t bytes, int64_t nn, int64_t vtot, bool mixed, bool pre) {
+        scratch = true;
         size_t off = 0;
         auto carve = [&](auto& buf, size_t count, bool need) {
             using T = std::remove_pointer_t<decltype(buf.p)>;
@@ -715,6 +730,7 @@ struct prism_csr {
     DevBuf<int16_t> sell_rel;
     std::vector<int32_t> dia_off;
     int64_t stotal{0};
+    int wmax{0};          // entries of the widest sliced-ELL slice
     bool all_diag{true};  // every row stores its diagonal entry
     DevBuf<double> val;
     Workspace ws;
@@ -739,6 +755,7 @@ struct MatRef {
     bool all_diag{true};                // every row stores its diagonal entry
     SgsCache* sgs{nullptr};             // the pattern's SGS plan (built on first use)
     const int32_t* sbase{nullptr};      // with srel: the base of each slice's slots
+    int wmax{0};                        // entries of the widest sliced-ELL slice
     // sets the DIA fields from a pattern's offsets (empty: no DIA view)
     void setDia(const int32_t* map, const std::vector<int32_t>& off) {
         ndia = map && !off.empty() ? (int)off.size() : 0;
@@ -842,6 +859,51 @@ bool traceEnabled() {
     }();
     return on;
 }
+
+// PRISM_KRYLOV_RESIDENT=0: the three-kernel iteration also where the resident kernel applies
+// (read per solve).  PRISM_KRYLOV_SPIN: polls of one of its waits at most.
+bool noResident() {
+    const char* e = std::getenv("PRISM_KRYLOV_RESIDENT");
+    return e && std::atoi(e) == 0;
+}
+unsigned residentSpin() {
+    const char* e = std::getenv("PRISM_KRYLOV_SPIN");
+    return e && std::atol(e) > 0 ? (unsigned)std::atol(e) : 1u << 20;
+}
+
+// Compute units that resident kernels of this process hold, per device.  Blocks of two such
+// kernels that cannot all run at once would wait for each other until their waits run out, so
+// a launch that does not fit beside those in flight is not made (the caller takes the
+// three-kernel iteration for that chunk).
+class ResidentTicket {
+    static std::atomic<int>& held(int device) {
+        static std::atomic<int> h[64];
+        return h[device & 63];
+    }
+    std::atomic<int>* at_{nullptr};
+    int blocks_{0};
+
+public:
+    bool take(int device, int blocks, int n_cu) {
+        give();
+        std::atomic<int>& h = held(device);
+        if (h.fetch_add(blocks) + blocks > n_cu) {
+            h.fetch_sub(blocks);
+            return false;
+        }
+        at_ = &h;
+        blocks_ = blocks;
+        return true;
+    }
+    void give() {
+        if (at_) at_->fetch_sub(blocks_);
+        at_ = nullptr;
+    }
+    ResidentTicket() = default;
+    ResidentTicket(const ResidentTicket&) = delete;
+    ResidentTicket& operator=(const ResidentTicket&) = delete;
+    ~ResidentTicket() { give(); }
+};
 
 bool graphsEnabled() {
     static const bool on = [] {
@@ -1126,6 +1188,30 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         }
         krylov_pack<T>(kv);
         bool three = !fiveKernels() && A.cscp;
+        // The resident kernel where the rows fit its registers (resident_plan); FP32 in the
+        // difference form only.
+        ResidentPlan plan;
+        ResidentView<T> rv{};
+        ResidentTicket ticket;
+        if (three && !w.scratch && (sizeof(T) == 8 || kv.diff) && !noResident())
+            plan = resident_plan<T>(A.n, dia, dia ? A.ndia : A.wmax, ctx->n_cu);
+        if (plan.blocks > 0) {
+            DevBuf<T>* pub;
+            if constexpr (sizeof(T) == 8) pub = &w.d_pub;
+            else pub = &w.f_pub;
+            const size_t words = resident_sums(plan.blocks);
+            pub->alloc(5 * (size_t)A.n);
+            w.slots.alloc(2 * words);
+            launch_resident_mark<T>(L, pub->p, pub->n);
+            launch_resident_mark<double>(L, reinterpret_cast<double*>(w.slots.p), w.slots.n);
+            rv.pub = pub->p;
+            rv.slots = w.slots.p;
+            rv.stale = w.slots.p + words;
+            rv.blocks = plan.blocks;
+            rv.rows = plan.rows;
+            rv.quota = 128;
+            rv.spin = residentSpin();
+        }
         auto setIter = [&](long long k) {  // buffers and rho slot of iteration k
             int q = (int)(k & 1);
             kv.par = q;
@@ -1196,6 +1282,18 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         int stalls = 0;       // forced updates in a row that did not lower the FP64 residual
         for (;;) {
             KrylovScalars s = pollScalars(ctx, w);
+            ticket.give();
+            if (s.stuck) {  // a wait of the resident kernel ran out: on from this x without it
+                if (traceEnabled()) std::fprintf(stderr, "krylov n=%d: resident kernel stuck\n", A.n);
+                plan.blocks = 0;
+                if constexpr (sizeof(T) == 4) launch_flush(L, A.n, x, kv.x);
+                launch_residual<T>(L, kv, b, x, w.r64.p, 0);
+                launch_reset_events(L, w.ks.p, true, false);
+                setIter(s.nit);
+                launch_seed<T>(L, kv, w.r64.p, 1);
+                enter(1);
+                continue;
+            }
             if (!s.done && !s.flag) {
                 if (s.rr < 0.25 * best) { best = s.rr; best_iter = s.nit; }
                 else if (s.nit - best_iter > window) {
@@ -1281,7 +1379,10 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             }
             last_iter = s.nit;
             last_rr = s.rr;
-            if (three) {
+            if (plan.blocks > 0 && ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu)) {
+                launch_resident<T>(L, kv, rv, plan);
+                std::swap(rv.slots, rv.stale);
+            } else if (three) {
                 for (int k = 0; k < chunk; ++k) {
                     setIter(s.nit + k);
                     launch_iteration3<T>(L, kv);
@@ -1458,6 +1559,7 @@ MatRef matOf(prism_eqn& e) {
     A.setDia(m->csr2dia.p, m->h.dia_off);
     A.sgs = &m->sgs;
     A.sbase = A.srel ? m->sell_base.p : nullptr;
+    A.wmax = m->wmax;
     return A;
 }
 
@@ -1526,6 +1628,7 @@ API int prism_ctx_create(int device, prism_ctx** out) {
         HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         HIPCHECK(hipHostMalloc((void**)&c->hks, sizeof(KrylovScalars), hipHostMallocDefault));
         c->scratch = static_cast<unsigned char*>(scratch_address(device));
+        HIPCHECK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device));
         *out = c.release();
     });
 }
@@ -1592,6 +1695,7 @@ API int prism_mesh_create(prism_ctx* ctx, const prism_mesh_desc* d, prism_mesh**
             m->dup_ptr.upload(h.dup_ptr, s);
         }
         m->gg_cells.upload(h.gg_cells, s);
+        m->wmax = widestSlice(h.sell_off);
         m->sell_off.upload(h.sell_off, s); m->sell_col.upload(h.sell_col, s); m->csr2sell.upload(h.csr2sell, s);
         if (!h.sell_rel.empty()) {
             m->sell_rel.upload(h.sell_rel, s);
@@ -2103,6 +2207,7 @@ API int prism_csr_create(prism_ctx* ctx, int64_t n, const int64_t* rp, const int
         a->sell_col.upload(sc, ctx->stream);
         a->csr2sell.upload(c2s, ctx->stream);
         a->stotal = (int64_t)sc.size();
+        a->wmax = widestSlice(so);
         std::vector<int16_t> rel;
         std::vector<int32_t> sbase;
         if (sellRelative(n, so, sc, rel, sbase)) {
@@ -2155,6 +2260,7 @@ API int prism_csr_bicgstab(prism_csr* a, const double* b, const double* xin, dou
         A.setDia(a->csr2dia.p, a->dia_off);
         A.all_diag = a->all_diag;
         A.sbase = A.srel ? a->sell_base.p : nullptr;
+        A.wmax = a->wmax;
         A.sgs = &a->sgs;
         StepOut so = krylovStep(a->ctx, a->ws, A, db.p, dx.p, *p);
         HIPCHECK(hipMemcpyAsync(xout, dx.p, a->n * sizeof(double), hipMemcpyDeviceToHost, a->ctx->stream));

@@ -1,0 +1,615 @@
+// resident.hip -- BiCGSTAB iterations of small and medium systems in one resident kernel.
+//
+// The three-kernel iteration (krylov.hip) of a system that fits the caches is bound by its
+// launches: a dependent launch costs 2.4 us and its prologue 2-3 us more, 14-20 us per
+// iteration, where the data would take 1-4 us (64^3 cells, 20 MB).  Here one launch runs up
+// to `quota` iterations of the same recurrences.  Each thread keeps R rows: their matrix entries
+// (values and element addresses) and their elements of x, r, r0, rhat, p, v, s and t stay in
+// registers from the first iteration to the last, so an iteration moves only p and s between
+// blocks, and the partial sums of its two reductions.  Per iteration, three kernels -> this
+// one: 200 rows FP64 14 -> 2.6 us, 16,384 rows FP64 15 -> 5.8 us, 82,944 rows of tetrahedra
+// FP32 17.5 -> 7.4 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us.  What
+// bounds it now is latency: four to five hops of 0.3-0.5 us between blocks per iteration, and
+// at two and three rows per thread the issue of the products (0.7 us per row and product).
+//
+// Exchange without barriers.  A word that another block waits for carries its own flag: it
+// holds the mark, a signalling NaN that no arithmetic produces (results are quiet NaNs), until
+// its owner stores the value; a reader polls until the word is not the mark.  Loads and
+// stores are relaxed atomics of agent scope, which all XCDs see without cache writebacks or
+// invalidations.  Per iteration k:
+//   sums (rhat, p_k), (r, r) -> the block's line; publish p_k
+//   V: A p_k (waits for the neighbours' p only); wait for the two totals; alpha;
+//      s = r - alpha v; publish s_k
+//   T: t = A s (waits for the neighbours' s only); sums (t,t), (t,s), (r0,s), (r0,t); wait for
+//      the four totals
+//   X: omega, beta, x, r, p_{k+1}
+// A block that has T's totals knows that every block has read s_k, the first two totals and
+// p_k: at the start of iteration k + 1 it marks its words of p_{k-1} and s_k and those sums
+// again (p_k stays: an event in iteration k + 1 hands it back to the host's state); T's sums
+// are marked after the next first totals.  Every word marked again is next polled after a
+// reduction that its owner took part in only when the marks were in memory (the s_waitcnt
+// before T's sums), so no reader sees an old value: p has three buffers, s, the sums and the
+// totals two.  Elements of the block's own rows are read from LDS instead.
+//
+// The reductions sum per thread, wave, block and then over the blocks in index order, with one
+// row per thread in exactly the order of the three-kernel iteration.  One block more than
+// the rows need does nothing else: a block that also has rows delays every reduction by its
+// own products (64^3: 12.2 us per iteration instead of 11.0).
+//
+// All blocks must run at the same time: at most one per compute unit.  Every wait is bounded
+// (rv.spin polls): if it runs out, ks->stuck tells the other blocks and the host, and the
+// launch ends; the host continues with the three-kernel iteration from the current x.
+#include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
+
+#include <algorithm>
+
+#include "../../include/prism_hip.h"
+#include "internal.h"
+#include "krylov.h"
+#include "resident.h"
+
+namespace prism_hip {
+
+namespace {
+
+constexpr int BS = RES_BS;
+constexpr int NW = BS / 64;
+
+template <typename T> struct Word;
+template <> struct Word<double> {
+    using U = unsigned long long;
+    static constexpr U MARK = 0x7FF4A11C0DE5EED1ull;  // a signalling NaN
+};
+template <> struct Word<float> {
+    using U = unsigned int;
+    static constexpr U MARK = 0x7FA5EED1u;
+};
+
+template <typename T>
+__device__ inline T asValue(typename Word<T>::U u) {
+    T v;
+    __builtin_memcpy(&v, &u, sizeof(T));
+    return v;
+}
+template <typename T>
+__device__ inline typename Word<T>::U asWord(T v) {
+    typename Word<T>::U u;
+    __builtin_memcpy(&u, &v, sizeof(T));
+    return u;
+}
+template <typename U>
+__device__ inline U peek(const U* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename U>
+__device__ inline void post(U* p, U v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Published vectors are reached through a buffer descriptor: one 32-bit offset per lane beside
+// scalar registers, and an offset past the end reads zero and stores nothing, without a
+// branch (FAR marks such offsets).  Cache policy 16 is the agent scope of peek and post.
+constexpr unsigned FAR = 0x80000000u;
+constexpr int AGENT = 16;
+using U2 = unsigned int __attribute__((ext_vector_type(2)));
+template <typename U>
+__device__ inline U bufPeek(__amdgpu_buffer_rsrc_t b, unsigned at, unsigned base) {
+    if constexpr (sizeof(U) == 8) {
+        const U2 v = __builtin_amdgcn_raw_buffer_load_b64(b, at, base, AGENT);
+        return (unsigned long long)v.y << 32 | v.x;
+    } else {
+        return __builtin_amdgcn_raw_buffer_load_b32(b, at, base, AGENT);
+    }
+}
+template <typename U>
+__device__ inline void bufPost(__amdgpu_buffer_rsrc_t b, unsigned at, unsigned base, U v) {
+    if constexpr (sizeof(U) == 8) {
+        const U2 w = {(unsigned)v, (unsigned)(v >> 32)};
+        __builtin_amdgcn_raw_buffer_store_b64(w, b, at, base, AGENT);
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b32(v, b, at, base, AGENT);
+    }
+}
+
+// Sums over the wavefront of K = 2 or 4 values at once, each with the additions of the
+// butterfly over lane distances 32, 16, 8, 4, 2, 1 (krylov.hip's waveSum: the same bits).  The
+// halves, and then the row pairs, of two values are swapped and added, which leaves each of
+// the K values on its own 64 / K lanes; DPP row rotations sum those: 7 additions for K = 4
+// instead of 24, and no moves through LDS.  The total of value k is in lane sumLane<K>(k).
+template <int CTRL>
+__device__ inline double rotAdd(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ inline double swapAdd32(double a, double b) {  // lanes 0-31: a's sums at distance 32, 32-63: b's
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ inline double swapAdd16(double a, double b) {  // even rows: a's sums at distance 16, odd rows: b's
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+template <int K>
+__device__ inline double waveSums(const double (&v)[K]) {
+    static_assert(K == 2 || K == 4);
+    double s = swapAdd32(v[0], v[1]);
+    if constexpr (K == 4) s = swapAdd16(s, swapAdd32(v[2], v[3]));  // rows 0 to 3: values 0, 2, 1, 3
+    else s = swapAdd16(s, s);
+    s = rotAdd<0x128>(s);  // row_ror:8
+    s = rotAdd<0x124>(s);  // row_ror:4
+    s = rotAdd<0x122>(s);  // row_ror:2
+    return rotAdd<0x121>(s);  // row_ror:1
+}
+template <int K>
+__device__ constexpr int sumLane(int k) {
+    return K == 2 ? 32 * k : 16 * (k == 1 ? 2 : k == 2 ? 1 : k);
+}
+__device__ inline double laneValue(double v, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double inOrder(const double* s) {  // the NW waves' sums
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t += s[i];
+    return t;
+}
+
+// blockIdx -> logical block: the blocks of one XCD own one contiguous range of rows.
+__device__ inline int logicalBlock(int nblk) {
+    const int b = blockIdx.x, q = nblk >> 3, r = nblk & 7, xcd = b & 7, idx = b >> 3;
+    return (xcd < r) ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
+}
+
+// A bounded wait: true while it may go on.  A wait that ran out, here or in another block
+// (looked up now and then), raises the block's flag.
+__device__ inline bool keepWaiting(unsigned& polls, unsigned limit, KrylovScalars* ks, int* fail) {
+    ++polls;
+    if (polls >= limit || ((polls & 255) == 0 && peek(&ks->stuck) != 0)) {
+        post(&ks->stuck, 1);
+        *fail = 1;
+        return false;
+    }
+    return true;
+}
+
+// Totals over all blocks of K values per thread, in two halves: postSums hands in this block's
+// sums (words slot[RES_LINE b + k] for block b, a cache line to each block), awaitTotals returns
+// the totals (block G's words); what is done between them hides the round trip.  The block without
+// rows (lb == G) gathers the sums and posts the totals that the others poll: every block
+// polling every sum took 3.1 us a round on 256 blocks, all of them reading the same lines
+// at once; one gather and one broadcast take 1.7 us.  The totals have a line for each XCD: 216
+// blocks polling one line lengthened an iteration of 48^3 rows from 8.2 to 9.5 us.  A
+// single block keeps both in LDS.
+// sh: K NW sums of waves, then the K totals.
+template <int K>
+__device__ inline void postSums(const double (&v)[K], unsigned long long* slot, int G, int lb, double* sh) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const double s = waveSums<K>(v);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (lane == sumLane<K>(k)) sh[k * NW + (tid >> 6)] = s;
+    __syncthreads();
+    if (G > 1 && lb < G && tid < K) post(&slot[RES_LINE * lb + tid], asWord(inOrder(sh + tid * NW)));
+}
+template <int K>
+__device__ inline bool awaitTotals(unsigned long long* slot, int G, int lb, unsigned limit, KrylovScalars* ks,
+                                   double* sh, int* fail, double (&out)[K]) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (G == 1) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) out[k] = inOrder(sh + k * NW);
+        return true;
+    }
+    unsigned polls = 0;
+    if (lb == G) {  // wave k gathers the sums k of up to RES_MAX_BLOCKS blocks
+        const int k = tid >> 6;
+        if (k < K) {
+            unsigned long long u[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) u[i] = lane + 64 * i < G ? peek(&slot[RES_LINE * (lane + 64 * i) + k]) : 0;
+            bool miss;
+            do {
+                miss = false;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (u[i] == Word<double>::MARK) {
+                        u[i] = peek(&slot[RES_LINE * (lane + 64 * i) + k]);
+                        miss |= u[i] == Word<double>::MARK;
+                    }
+            } while (miss && keepWaiting(polls, limit, ks, fail));
+            const double part[4] = {asValue<double>(u[0]), asValue<double>(u[1]), asValue<double>(u[2]),
+                                    asValue<double>(u[3])};
+            const double s = waveSums<4>(part);
+            double t = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t += laneValue(s, sumLane<4>(i));
+            if (lane < RES_COPIES) post(&slot[RES_LINE * (G + lane) + k], asWord(t));
+            if (lane == 0) sh[K * NW + k] = t;
+        }
+    } else if (tid < K) {
+        const unsigned long long* total = &slot[RES_LINE * (G + (int)(blockIdx.x & (RES_COPIES - 1))) + tid];
+        unsigned long long u = peek(total);
+        while (u == Word<double>::MARK && keepWaiting(polls, limit, ks, fail)) u = peek(total);
+        sh[K * NW + tid] = asValue<double>(u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) out[k] = sh[K * NW + k];
+    return *fail == 0;
+}
+
+// FP64: plain row products; FP32: the difference form (matRow in krylov.hip; the diagonal
+// coefficient holds the row sum, or zero where the matrix has zero row sums).
+template <typename T, bool DIA, int W, int R>
+__global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv) {
+    using U = typename Word<T>::U;
+    constexpr U MARK = Word<T>::MARK;
+    constexpr bool DIFF = sizeof(T) == 4;
+    __shared__ T own[2][R * BS + 1];  // this block's p and s, and a zero
+    __shared__ double shA[2 * NW + 2], shC[4 * NW + 4];
+    __shared__ int fail;
+    KrylovScalars* ks = kv.ks;
+    const int tid = threadIdx.x, G = rv.blocks, n = kv.n;
+    // the last block has no rows: it gathers the sums of the others (a single block: none does)
+    const int lb = (int)blockIdx.x < G ? logicalBlock(G) : G;
+    const int r0 = lb < G ? lb * rv.rows : n, r1 = min(r0 + rv.rows, n);
+    // rows of this wave: j < live holds one in some lane
+    const int live = __builtin_amdgcn_readfirstlane(max(0, (r1 - r0 - (tid & ~63) + BS - 1) / BS));
+    if (ks->done | ks->flag | ks->stuck) return;  // the same value in every thread of the grid
+    if (tid == 0) {
+        fail = 0;
+        own[0][R * BS] = own[1][R * BS] = T(0);
+    }
+    if (tid < RES_LINE * (lb < G ? 1 : RES_COPIES)) post(&rv.stale[RES_LINE * lb + tid], Word<double>::MARK);
+
+    // this thread's rows r0 + tid + j BS; at[j][k]: where entry k's element is, as a byte offset
+    // into own[] (this block's), or FAR + its byte offset in the published vector
+    T a[R][W], x[R], r[R], z[R], h[R], p[R], v[R], s[R], t[R];
+    unsigned at[R][W];
+    auto rowOf = [&](int j) { return r0 + tid + j * BS; };
+    auto mine = [&](int j) { return (unsigned)(tid + j * BS) * (unsigned)sizeof(T); };
+    auto rowAt = [&](int j) { return rowOf(j) < r1 ? (unsigned)rowOf(j) * (unsigned)sizeof(T) : FAR; };
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int row = rowOf(j);
+        const bool ok = row < r1;
+        x[j] = ok ? kv.x[row] : T(0);
+        r[j] = ok ? kv.r[row] : T(0);
+        z[j] = ok ? kv.r0[row] : T(0);
+        h[j] = ok ? kv.rhat[row] : T(0);
+        p[j] = ok ? kv.p_new[row] : T(0);
+        v[j] = s[j] = t[j] = T(0);
+        int o = 0, w = 0;
+        if (!DIA && ok) {
+            o = kv.soff[row >> 6];
+            w = (kv.soff[(row >> 6) + 1] - o) >> 6;
+        }
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            int c = row;  // a missing entry: coefficient zero, the row's own element
+            T e = T(0);
+            if constexpr (DIA) {
+                if (ok && k < kv.ndia && (unsigned)(row + kv.doff[k]) < (unsigned)n) {
+                    c = row + kv.doff[k];
+                    e = kv.sval[(int64_t)k * n + row];
+                }
+            } else if (k < w) {
+                const int q = (int)sellPos(o, w, k, row & 63);
+                c = kv.srel ? row + kv.sbase[(o >> 6) + k] + (int)kv.srel[q] : kv.scol[q];
+                e = kv.sval[q];
+            }
+            if (DIFF && kv.diff == 2 && c == row) e = T(0);
+            a[j][k] = e;
+            const int l = ok ? c - r0 : 0;
+            at[j][k] = (unsigned)l < (unsigned)rv.rows ? (unsigned)l * (unsigned)sizeof(T)
+                                                        : FAR + (unsigned)c * (unsigned)sizeof(T);
+        }
+    }
+    unsigned long long wants = 0;  // bit j W + k: some lane of the wave reads entry k of row j from another block
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int k = 0; k < W; ++k)
+            if (__ballot(at[j][k] >= FAR)) wants |= 1ull << (j * W + k);
+    const __amdgpu_buffer_rsrc_t pub =
+        __builtin_amdgcn_make_buffer_rsrc(rv.pub, 0, 5 * n * (int)sizeof(T), 0x00020000);
+    const unsigned bytes = (unsigned)n * (unsigned)sizeof(T);  // of one published vector
+    const bool mixed = kv.mixed != 0, pc = kv.precond != 0;
+    const double tol2 = ks->tol2, ref2 = ks->delta2 * ks->rr_ref, tiny = ks->breakdown * ks->r0n;
+    double rho = ks->rho[kv.par], alpha = ks->alpha, omega = ks->omega;
+    double rho_old = 0.0, beta = 0.0, tt = 0.0, ts = 0.0, rp = 0.0, rr = 0.0;
+    const long long iter0 = ks->iter, maxit = ks->maxit;
+    int done = 0, flag = 0, m = 0;
+    __syncthreads();  // fail
+
+    // y = A w for the vector published at byte `base` (this block's elements in own[q]).  An
+    // element that is not there yet reads as the mark and makes the row's sum a NaN: only then
+    // are the elements looked at one by one.
+    auto product = [&](unsigned base, int q, const T (&w)[R], T (&y)[R]) {
+        const char* mem = reinterpret_cast<const char*>(own[q]);
+        U u[R][W];
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int k = 0; k < W; ++k) {
+                asm volatile("" : "+v"(at[j][k]));  // no copies of what follows kept per iteration
+                u[j][k] = U(0);
+                if (wants >> (j * W + k) & 1) u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
+            }
+        unsigned polls = 0;
+        for (;;) {
+            bool nan = false;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                if (j >= live) continue;
+                T sum = T(0);
+#pragma unroll
+                for (int k = 0; k < W; ++k) {
+                    // one of the two is zero: own[q] ends with one, the buffer read was out of range
+                    const U l = asWord(*reinterpret_cast<const T*>(mem + min(at[j][k], (unsigned)(R * BS * sizeof(T)))));
+                    const T e = asValue<T>(l | u[j][k]);
+                    if (DIFF) sum += a[j][k] * (at[j][k] == mine(j) ? w[j] : e - w[j]);
+                    else sum += a[j][k] * e;
+                }
+                y[j] = sum;
+                nan |= sum != sum;
+            }
+            if (!nan) break;
+            bool miss = false;
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+#pragma unroll
+                for (int k = 0; k < W; ++k)
+                    if (u[j][k] == MARK) {
+                        miss = true;
+                        u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
+                    }
+            if (!miss || !keepWaiting(polls, rv.spin, ks, &fail)) break;
+        }
+    };
+    auto keep = [&](int q, const T (&w)[R]) {
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (j < live) own[q][tid + j * BS] = w[j];
+    };
+    auto publish = [&](unsigned base, const T (&w)[R]) {
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (j < live) bufPost(pub, rowAt(j), base, asWord(w[j]));
+    };
+    auto mark = [&](unsigned base) {
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (j < live) bufPost(pub, rowAt(j), base, MARK);
+    };
+    auto sBase = [&](int k) { return (unsigned)(3 + (k & 1)) * bytes; };
+    // words of a block's line: the two sums of each parity, then the four of each parity; the
+    // summing block's line (the last one) holds the totals
+    auto slotA = [&](int k) { return rv.slots + (k & 1) * 2; };
+    auto slotC = [&](int k) { return rv.slots + 4 + (k & 1) * 4; };
+    auto markSums = [&](unsigned long long* sl, int words) {
+        if (G > 1 && tid < (lb < G ? words : words * RES_COPIES))
+            post(&sl[RES_LINE * (lb + tid / words) + tid % words], Word<double>::MARK);
+    };
+
+    double acc[2] = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        acc[0] += (double)h[j] * (double)p[j];
+        acc[1] += (double)r[j] * (double)r[j];
+    }
+    unsigned pm = 0, pm_old = 2;  // m modulo 3, and of the previous iteration
+    for (;;) {
+        keep(0, p);
+        postSums<2>(acc, slotA(m), G, lb, shA);
+        publish(pm * bytes, p);  // a single block's, too: p_{k-1} is read back at the end
+        if (m > 0) {  // every block has read these
+            if (m > 1 && G > 1) mark((pm_old == 0 ? 2 : pm_old - 1) * bytes);
+            if (G > 1) mark(sBase(m - 1));
+            markSums(slotA(m - 1), 2);
+        }
+        T vn[R] = {};
+        if (live) product(pm * bytes, 0, p, vn);
+        double red[2];
+        if (!awaitTotals<2>(slotA(m), G, lb, rv.spin, ks, shA, &fail, red)) return;
+        rp = red[0];
+        rr = red[1];
+        if (m > 0) markSums(slotC(m - 1), 4);
+        // convergence and events, in the order of the three-kernel iteration
+        if (!(rr == rr)) done = 3;
+        else if (mixed) {
+            if (rr <= tol2 || rr <= ref2 || iter0 + m >= maxit) flag = 1;
+        } else if (rr <= tol2) done = 1;
+        else if (iter0 + m >= maxit) done = 2;
+        if (!done && !flag) {
+            if (!(rp == rp) || !(rho == rho)) done = 3;
+            else if (fabs(rho) < tiny) flag = 2;
+        }
+        if (done || flag || m >= rv.quota) break;
+        alpha = rho / rp;
+        const T al = (T)alpha;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            if (j >= live) continue;
+            v[j] = vn[j];
+            s[j] = r[j] - al * v[j];
+        }
+        if (G > 1) publish(sBase(m), s);
+        keep(1, s);
+        __syncthreads();
+        if (live) product(sBase(m), 1, s, t);
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            if (j >= live) continue;
+            const double td = (double)t[j], sd = (double)s[j], zd = (double)z[j];
+            d[0] += td * td;
+            d[1] += td * sd;
+            d[2] += zd * sd;
+            d[3] += zd * td;
+        }
+        // the marks stored since the last of these sums are in memory before this block's are
+        if (G > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        postSums<4>(d, slotC(m), G, lb, shC);
+        double tot[4];
+        if (!awaitTotals<4>(slotC(m), G, lb, rv.spin, ks, shC, &fail, tot)) return;
+        tt = tot[0];
+        ts = tot[1];
+        omega = tt > 0.0 ? ts / tt : 0.0;
+        const double rho1 = tot[2] - omega * tot[3];
+        beta = (rho1 / rho) * (alpha / omega);
+        const T w = (T)omega, b = (T)beta;
+        acc[0] = acc[1] = 0.0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            if (j >= live) continue;
+            const T di = pc && rowOf(j) < r1 ? kv.dinv[rowOf(j)] : T(1);
+            const T yi = pc ? di * p[j] : p[j], zi = pc ? di * s[j] : s[j];
+            x[j] = x[j] + (al * yi + w * zi);
+            r[j] = s[j] - w * t[j];
+            p[j] = r[j] + b * (p[j] - w * v[j]);
+            const double rd = (double)r[j];
+            acc[0] += (double)h[j] * (double)p[j];
+            acc[1] += rd * rd;
+        }
+        rho_old = rho;
+        rho = rho1;
+        ++m;
+        pm_old = pm;
+        pm = pm == 2 ? 0 : pm + 1;
+    }
+
+    // the state as the three-kernel iteration keeps it: p_k and rho_k in slot k & 1, p_{k-1},
+    // v_{k-1} and rho_{k-1} in the other one
+    const bool even = (m & 1) == 0;
+    T* pk = even ? kv.p_new : kv.p_old;
+    T* pl = even ? kv.p_old : kv.p_new;
+    T* vl = even ? kv.v_old : kv.v_new;
+    if (m > 0) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int row = rowOf(j);
+            if (row >= r1) continue;
+            kv.x[row] = x[j];
+            kv.r[row] = r[j];
+            pk[row] = p[j];
+            pl[row] = asValue<T>(bufPeek<U>(pub, rowAt(j), pm_old * bytes));
+            vl[row] = v[j];
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        mark(pm_old * bytes);
+    }
+    mark(pm * bytes);
+    if (lb == 0)  // the partial sums that the three-kernel iteration's V reduces
+        for (int i = tid; i < kv.G; i += BS) {
+            kv.part_x[i] = i == 0 ? rp : 0.0;
+            kv.part_x[kv.G + i] = i == 0 ? rr : 0.0;
+        }
+    if (lb == 0 && tid == 0) {
+        ks->rr = rr;
+        if (m > 0) {
+            const int q = kv.par ^ (m & 1);
+            ks->rho[q] = rho;
+            ks->rho[q ^ 1] = rho_old;
+            ks->alpha = alpha;
+            ks->omega = omega;
+            ks->beta = beta;
+            ks->tt = tt;
+            ks->ts = ts;
+            ks->iter = iter0 + m;
+            ks->nit += m;
+        }
+        ks->r0v = rp;
+        if (done) ks->done = done;
+        else if (flag) ks->flag = flag;
+    }
+}
+
+template <typename T>
+__global__ void k_mark(T* p, size_t count) {
+    using U = typename Word<T>::U;
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) reinterpret_cast<U*>(p)[i] = Word<T>::MARK;
+}
+
+template <typename T, bool DIA, int W, int R>
+void launchOne(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv) {
+    PRISM_LAUNCH(sizeof(T) == 8 ? "bicgstab_resident_f64" : "bicgstab_resident_f32", (k_resident<T, DIA, W, R>),
+                 rv.blocks + (rv.blocks > 1 ? 1 : 0), BS, kv, rv);
+}
+
+template <typename T, bool DIA, int W>
+void launchR(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, int R) {
+    switch (R) {
+    case 1: launchOne<T, DIA, W, 1>(L, kv, rv); break;
+    case 2: launchOne<T, DIA, W, 2>(L, kv, rv); break;
+    case 3: launchOne<T, DIA, W, 3>(L, kv, rv); break;
+    case 4:
+        if constexpr (sizeof(T) == 4) launchOne<T, DIA, W, 4>(L, kv, rv);
+        break;
+    default: throw Error(PRISM_ERR_RUNTIME, "resident BiCGSTAB: no kernel for this many rows per thread");
+    }
+}
+
+}  // namespace
+
+// R rows per thread at most, as few as the blocks allow (one less than the compute units: one
+// block sums).  With one row per thread, the rows per block of the three-kernel iteration: the
+// sums are then formed in the same order, and the iterates are the same bits.  With more, as
+// many blocks as there can be, so that the rows of a block, and with them an iteration's
+// work, are fewest.
+template <typename T>
+ResidentPlan resident_plan(int64_t n, bool dia, int wmax, int n_cu) {
+    ResidentPlan p;
+    const int W = wmax <= 5 ? 5 : wmax <= 8 ? (dia && wmax <= 7 ? 7 : 8) : wmax <= 16 && !dia ? 16 : 0;
+    const int most = std::min(n_cu - 1, RES_MAX_BLOCKS);
+    if (!W || n < 1 || most < 1) return p;
+    const int rmax = W == 16 ? 1 : sizeof(T) == 4 ? 4 : 3;
+    int spb = 0;
+    krylov_grid(n, &spb);
+    int64_t rows = (int64_t)spb * 64;
+    if (n > (int64_t)most * RES_BS) rows = ((n + most - 1) / most + 63) / 64 * 64;
+    const int64_t R = (rows + RES_BS - 1) / RES_BS;
+    if (R > rmax) return p;
+    p.blocks = (int)((n + rows - 1) / rows);
+    p.rows = (int)rows;
+    p.R = (int)R;
+    p.W = W;
+    return p;
+}
+
+template <typename T>
+void launch_resident_mark(const Launch& L, T* p, size_t count) {
+    if (count) PRISM_LAUNCH("resident_mark", k_mark<T>, (int)((count + 255) / 256), 256, p, count);
+}
+
+template <typename T>
+void launch_resident(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, const ResidentPlan& plan) {
+    if (kv.ndia) {
+        if (plan.W == 5) launchR<T, true, 5>(L, kv, rv, plan.R);
+        else if (plan.W == 7) launchR<T, true, 7>(L, kv, rv, plan.R);
+        else launchR<T, true, 8>(L, kv, rv, plan.R);
+    } else {
+        if (plan.W == 5) launchR<T, false, 5>(L, kv, rv, plan.R);
+        else if (plan.W == 8) launchR<T, false, 8>(L, kv, rv, plan.R);
+        else launchOne<T, false, 16, 1>(L, kv, rv);
+    }
+}
+
+template ResidentPlan resident_plan<double>(int64_t, bool, int, int);
+template ResidentPlan resident_plan<float>(int64_t, bool, int, int);
+template void launch_resident_mark<double>(const Launch&, double*, size_t);
+template void launch_resident_mark<float>(const Launch&, float*, size_t);
+template void launch_resident<double>(const Launch&, const KView<double>&, const ResidentView<double>&,
+                                      const ResidentPlan&);
+template void launch_resident<float>(const Launch&, const KView<float>&, const ResidentView<float>&,
+                                     const ResidentPlan&);
+
+}  // namespace prism_hip

@@ -1,0 +1,120 @@
+"""The resident BiCGSTAB kernel (resident.hip) against the three-kernel iteration and against
+exact solutions: with one row per thread both form every sum in the same order, so the
+solutions are the same bits; with more, each solution satisfies the system."""
+import threading
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import prism_amd as P
+
+pytestmark = pytest.mark.gpu
+
+
+def scattered(n, row, seed=3):
+    """Strictly diagonally dominant, nonsymmetric, `row` scattered off-diagonals a row at most."""
+    rng = np.random.default_rng(seed)
+    A = sp.coo_matrix((rng.uniform(-1.0, 0.3, n * row), (np.repeat(np.arange(n), row), rng.integers(0, n, n * row))),
+                      shape=(n, n)).tocsr()
+    A.setdiag(0.0)
+    A.setdiag(1.1 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)
+    A.sort_indices()
+    return A
+
+
+def diagonals(n, offsets, seed=4):
+    """The same on the given diagonals."""
+    rng = np.random.default_rng(seed)
+    A = sp.diags([rng.uniform(-1.0, 0.3, n - abs(o)) for o in offsets], offsets, shape=(n, n), format="csr")
+    A = (A + sp.diags(1.1 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)).tocsr()
+    A.sort_indices()
+    return A
+
+
+def matrix(hip, A):
+    return P.Matrix(hip, A.indptr, A.indices, A.data)
+
+
+def solve(hip, A, monkeypatch, resident, **kw):
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "1" if resident else "0")
+    b = np.random.default_rng(9).standard_normal(A.shape[0])
+    hip.set_timing(True)
+    hip.reset_timing()
+    out = []
+    x = P.solver.BiCGSTAB(tol=1e-12, max_iters=2000, **kw).step(matrix(hip, A), np.zeros(A.shape[0]), b, out)
+    names = set(hip.kernel_stats())
+    hip.set_timing(False)
+    return x, b, out[0], any(k.startswith("bicgstab_resident") for k in names)
+
+
+SYSTEMS = {
+    "sell5_1": scattered(1, 1), "sell5_63": scattered(63, 3), "sell5_512": scattered(512, 4),
+    "sell5_513": scattered(513, 4), "sell8_640": scattered(640, 7), "sell8_9001": scattered(9001, 7),
+    "sell16_700": scattered(700, 14), "sell16_6400": scattered(6400, 12),
+    "dia3_513": diagonals(513, (-1, 1)), "dia5_1600": diagonals(1600, (-40, -1, 1, 40)),
+    "dia7_4095": diagonals(4095, (-195, -13, -1, 1, 13, 195)),
+    "dia8_2049": diagonals(2049, (-500, -20, -3, -1, 1, 20, 500)),
+}
+
+
+@pytest.mark.parametrize("precision,precond", [("fp64", None), ("fp64", "jacobi"), ("fp32", None), ("fp32", "jacobi")])
+@pytest.mark.parametrize("name", list(SYSTEMS))
+def test_same_bits_as_three_kernels(hip, monkeypatch, name, precision, precond):
+    print(f"case resident {name} {precision} {precond}", flush=True)
+    A = SYSTEMS[name]
+    x1, b, r1, used1 = solve(hip, A, monkeypatch, True, precision=precision, precond=precond)
+    x0, _, r0, used0 = solve(hip, A, monkeypatch, False, precision=precision, precond=precond)
+    assert not used0 and (used1 or r1.krylov_iters == 0)
+    np.testing.assert_array_equal(x1, x0)
+    assert (r1.krylov_iters, r1.refinements, r1.restarts) == (r0.krylov_iters, r0.refinements, r0.restarts)
+    # ||b - A x|| <= 1e-12 ||b|| recomputed by the library, to twice that here (other rounding)
+    assert np.linalg.norm(b - A @ x1) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n,precision", [(255 * 512 + 1, "fp64"), (262144, "fp64"), (255 * 1536, "fp64"),
+                                         (255 * 512 + 1, "fp32"), (400001, "fp32"), (255 * 2048, "fp32")])
+def test_several_rows_per_thread(hip, monkeypatch, n, precision):
+    print(f"case resident rows {n} {precision}", flush=True)
+    A = diagonals(n, (-4096, -64, -1, 1, 64, 4096))
+    x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision)
+    assert used
+    assert r.krylov_rel_residual <= 1e-12
+    assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_wait_that_runs_out_falls_back(hip, monkeypatch, precision):
+    """One poll per wait: the blocks give up at their first wait, and the solve goes on with the
+    three-kernel iteration."""
+    print(f"case resident spin {precision}", flush=True)
+    monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
+    A = scattered(9001, 7)
+    x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision)
+    assert used and r.krylov_rel_residual <= 1e-12
+    assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+
+
+def test_two_threads_share_the_device(hip, monkeypatch):
+    """Two contexts solve at once; together their blocks exceed the device, so one of them takes
+    the three-kernel iteration now and then: the same bits either way."""
+    print("case resident two threads", flush=True)
+    monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
+    A = diagonals(100000, (-2000, -50, -1, 1, 50, 2000))
+    b = np.random.default_rng(1).standard_normal(A.shape[0])
+    alone = P.solver.BiCGSTAB(tol=1e-12).step(matrix(hip, A), np.zeros(A.shape[0]), b)
+    out = {}
+
+    def work(k):
+        be = P.Backend.hip(0)
+        M = matrix(be, A)
+        out[k] = [P.solver.BiCGSTAB(tol=1e-12).step(M, np.zeros(A.shape[0]), b) for _ in range(3)]
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for k in range(2):
+        for x in out[k]:
+            np.testing.assert_array_equal(x, alone)
