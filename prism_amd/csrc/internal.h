@@ -176,6 +176,11 @@ void launch_grad_ls(const Launch& L, const DMesh& m, const DScalar& s, double* g
 void launch_grad_ls3(const Launch& L, const DMesh& m, const DScalar (&s)[3], double* const (&g)[3]);
 void launch_grad_gg_level(const Launch& L, const DMesh& m, const DScalar& s, const int32_t* cells,
                           int32_t count, double* gx, double* gy, double* gz);
+// The whole sweep at once (cells of at most gg_sweep_faces() faces); off: the levels' offsets, on
+// the device; lower, terms: scratch of gg_sweep_faces() n and 7 gg_sweep_faces() n words.
+int gg_sweep_faces();
+void launch_grad_gg_sweep(const Launch& L, const DMesh& m, const DScalar& s, const int32_t* cells, const int32_t* off,
+                          int32_t levels, int32_t* lower, double* terms, double* gx, double* gy, double* gz);
 void launch_assemble(const Launch& L, const DMesh& m, const DEquation& e, int32_t relax, double urf);
 void launch_relax(const Launch& L, const DMesh& m, double* A, double* b, const double* phi, double urf);
 void launch_ref_cell(const Launch& L, const DMesh& m, double* A, double* b, int32_t cell, double ref);
