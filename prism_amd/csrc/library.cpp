@@ -189,6 +189,7 @@ struct SgsPlan {
     DevBuf<int32_t> soff, scol, emap;   // off-diagonals: slice offsets, position columns, CSR index
     DevBuf<int32_t> dmap;               // position -> CSR index of its diagonal entry
     int64_t slots{0};
+    int wmax{0};                        // entries of the widest slice
 };
 struct SgsCache {
     std::unique_ptr<SgsPlan> plan;
@@ -505,6 +506,8 @@ struct Workspace {  // Krylov buffers of one equation, allocated on first solve
     struct Sgs {
         DevBuf<double> sval, d, dinv, x, b, r, r0, p, v, y, s, z, t, e, part_x, part_v, part_t;
         DevBuf<SgsState> st;
+        DevBuf<double> pub;  // resident kernel: exchanged words, sums
+        DevBuf<unsigned long long> lines;
     } sgs;
     // Captured pairs of iterations (even/odd start) per precision, keyed by the kernel
     // arguments they were captured with.
@@ -896,6 +899,8 @@ unsigned residentSpin() {
     return e && std::atol(e) > 0 ? (unsigned)std::atol(e) : 1u << 20;
 }
 
+constexpr int RESIDENT_QUOTA = 128;  // iterations of one resident launch
+
 // Compute units that resident kernels of this process hold, per device.  Blocks of two such
 // kernels that cannot all run at once would wait for each other until their waits run out, so
 // a launch that does not fit beside those in flight is not made (the caller takes the
@@ -993,6 +998,7 @@ std::unique_ptr<SgsPlan> buildSgsPlan(prism_ctx* ctx, const MatRef& A) {
     plan->nc = lay.nc;
     plan->cptr = lay.cptr;
     plan->slots = (int64_t)lay.scol.size();
+    plan->wmax = widestSlice(lay.soff);
     plan->perm.upload(lay.perm, ctx->stream);
     plan->soff.upload(lay.soff, ctx->stream);
     plan->scol.upload(lay.scol, ctx->stream);
@@ -1054,16 +1060,46 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     StepOut out;
     long long k = 0, base = 0;  // base: Eigen restarts its iteration count at the first restart
     int fresh = 1, chunk = 4;
+    SgsResidentView rv{};
+    ResidentTicket ticket;
+    bool resident = !noResident() && sgs_resident_fits(n, P.wmax, ctx->n_cu, &rv.blocks);
+    if (resident) {
+        const size_t words = resident_sums(rv.blocks);
+        W.pub.alloc(6 * (size_t)n);
+        W.lines.alloc(2 * words);
+        launch_resident_mark<double>(L, W.pub.p, W.pub.n);
+        launch_resident_mark<double>(L, reinterpret_cast<double*>(W.lines.p), W.lines.n);
+        rv.pub = W.pub.p;
+        rv.line = W.lines.p;
+        rv.stale = W.lines.p + words;
+        rv.spin = residentSpin();
+    }
     for (;;) {
-        const long long todo = std::min<long long>(chunk, maxit - (k - base));
+        const bool here = resident && ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
+        const long long todo = std::min<long long>(here ? RESIDENT_QUOTA : chunk, maxit - (k - base));
         if (todo <= 0) {
             out.done = 2;
             out.iters = k - base;
             break;
         }
-        for (long long j = 0; j < todo; ++j) launch_sgs_iteration(L, V, k + j, j == 0 ? fresh : 0);
+        if (here) {
+            rv.quota = (int)todo;
+            launch_sgs_resident(L, V, rv, P.wmax, k, fresh);
+            std::swap(rv.line, rv.stale);
+        } else {
+            for (long long j = 0; j < todo; ++j) launch_sgs_iteration(L, V, k + j, j == 0 ? fresh : 0);
+        }
         fresh = 0;
         const SgsState s = poll();
+        ticket.give();
+        if (s.stuck) {  // a wait of the resident kernel ran out: on from this x without it
+            resident = false;
+            h.s[0] = h.s[1];  // the start state at either parity
+            HIPCHECK(hipMemcpyAsync(W.st.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
+            launch_sgs_seed(L, V, true);
+            fresh = 1;
+            continue;
+        }
         if (s.done) {
             out.done = s.done;
             out.iters = s.k_event - base;
@@ -1234,7 +1270,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             rv.stale = w.slots.p + words;
             rv.blocks = plan.blocks;
             rv.rows = plan.rows;
-            rv.quota = 128;
+            rv.quota = RESIDENT_QUOTA;
             rv.spin = residentSpin();
         }
         auto setIter = [&](long long k) {  // buffers and rho slot of iteration k

@@ -45,6 +45,7 @@
 #include <algorithm>
 
 #include "../../include/prism_hip.h"
+#include "exchange.h"
 #include "internal.h"
 #include "krylov.h"
 #include "resident.h"
@@ -56,103 +57,6 @@ namespace {
 constexpr int BS = RES_BS;
 constexpr int NW = BS / 64;
 
-template <typename T> struct Word;
-template <> struct Word<double> {
-    using U = unsigned long long;
-    static constexpr U MARK = 0x7FF4A11C0DE5EED1ull;  // a signalling NaN
-};
-template <> struct Word<float> {
-    using U = unsigned int;
-    static constexpr U MARK = 0x7FA5EED1u;
-};
-
-template <typename T>
-__device__ inline T asValue(typename Word<T>::U u) {
-    T v;
-    __builtin_memcpy(&v, &u, sizeof(T));
-    return v;
-}
-template <typename T>
-__device__ inline typename Word<T>::U asWord(T v) {
-    typename Word<T>::U u;
-    __builtin_memcpy(&u, &v, sizeof(T));
-    return u;
-}
-template <typename U>
-__device__ inline U peek(const U* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename U>
-__device__ inline void post(U* p, U v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Published vectors are reached through a buffer descriptor: one 32-bit offset per lane beside
-// scalar registers, and an offset past the end reads zero and stores nothing, without a
-// branch (FAR marks such offsets).  Cache policy 16 is the agent scope of peek and post.
-constexpr unsigned FAR = 0x80000000u;
-constexpr int AGENT = 16;
-using U2 = unsigned int __attribute__((ext_vector_type(2)));
-template <typename U>
-__device__ inline U bufPeek(__amdgpu_buffer_rsrc_t b, unsigned at, unsigned base) {
-    if constexpr (sizeof(U) == 8) {
-        const U2 v = __builtin_amdgcn_raw_buffer_load_b64(b, at, base, AGENT);
-        return (unsigned long long)v.y << 32 | v.x;
-    } else {
-        return __builtin_amdgcn_raw_buffer_load_b32(b, at, base, AGENT);
-    }
-}
-template <typename U>
-__device__ inline void bufPost(__amdgpu_buffer_rsrc_t b, unsigned at, unsigned base, U v) {
-    if constexpr (sizeof(U) == 8) {
-        const U2 w = {(unsigned)v, (unsigned)(v >> 32)};
-        __builtin_amdgcn_raw_buffer_store_b64(w, b, at, base, AGENT);
-    } else {
-        __builtin_amdgcn_raw_buffer_store_b32(v, b, at, base, AGENT);
-    }
-}
-
-// Sums over the wavefront of K = 2 or 4 values at once, each with the additions of the
-// butterfly over lane distances 32, 16, 8, 4, 2, 1 (krylov.hip's waveSum: the same bits).  The
-// halves, and then the row pairs, of two values are swapped and added, which leaves each of
-// the K values on its own 64 / K lanes; DPP row rotations sum those: 7 additions for K = 4
-// instead of 24, and no moves through LDS.  The total of value k is in lane sumLane<K>(k).
-template <int CTRL>
-__device__ inline double rotAdd(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
-    return v + __hiloint2double(hi, lo);
-}
-__device__ inline double swapAdd32(double a, double b) {  // lanes 0-31: a's sums at distance 32, 32-63: b's
-    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
-}
-__device__ inline double swapAdd16(double a, double b) {  // even rows: a's sums at distance 16, odd rows: b's
-    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
-}
-template <int K>
-__device__ inline double waveSums(const double (&v)[K]) {
-    static_assert(K == 2 || K == 4);
-    double s = swapAdd32(v[0], v[1]);
-    if constexpr (K == 4) s = swapAdd16(s, swapAdd32(v[2], v[3]));  // rows 0 to 3: values 0, 2, 1, 3
-    else s = swapAdd16(s, s);
-    s = rotAdd<0x128>(s);  // row_ror:8
-    s = rotAdd<0x124>(s);  // row_ror:4
-    s = rotAdd<0x122>(s);  // row_ror:2
-    return rotAdd<0x121>(s);  // row_ror:1
-}
-template <int K>
-__device__ constexpr int sumLane(int k) {
-    return K == 2 ? 32 * k : 16 * (k == 1 ? 2 : k == 2 ? 1 : k);
-}
-__device__ inline double laneValue(double v, int lane) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-    return __hiloint2double(hi, lo);
-}
 __device__ inline double inOrder(const double* s) {  // the NW waves' sums
     double t = 0.0;
 #pragma unroll
@@ -164,18 +68,6 @@ __device__ inline double inOrder(const double* s) {  // the NW waves' sums
 __device__ inline int logicalBlock(int nblk) {
     const int b = blockIdx.x, q = nblk >> 3, r = nblk & 7, xcd = b & 7, idx = b >> 3;
     return (xcd < r) ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-}
-
-// A bounded wait: true while it may go on.  A wait that ran out, here or in another block
-// (looked up now and then), raises the block's flag.
-__device__ inline bool keepWaiting(unsigned& polls, unsigned limit, KrylovScalars* ks, int* fail) {
-    ++polls;
-    if (polls >= limit || ((polls & 255) == 0 && peek(&ks->stuck) != 0)) {
-        post(&ks->stuck, 1);
-        *fail = 1;
-        return false;
-    }
-    return true;
 }
 
 // Totals over all blocks of K values per thread, in two halves: postSums hands in this block's
@@ -222,7 +114,7 @@ __device__ inline bool awaitTotals(unsigned long long* slot, int G, int lb, unsi
                         u[i] = peek(&slot[RES_LINE * (lane + 64 * i) + k]);
                         miss |= u[i] == Word<double>::MARK;
                     }
-            } while (miss && keepWaiting(polls, limit, ks, fail));
+            } while (miss && keepWaiting(polls, limit, &ks->stuck, fail));
             const double part[4] = {asValue<double>(u[0]), asValue<double>(u[1]), asValue<double>(u[2]),
                                     asValue<double>(u[3])};
             const double s = waveSums<4>(part);
@@ -235,7 +127,7 @@ __device__ inline bool awaitTotals(unsigned long long* slot, int G, int lb, unsi
     } else if (tid < K) {
         const unsigned long long* total = &slot[RES_LINE * (G + (int)(blockIdx.x & (RES_COPIES - 1))) + tid];
         unsigned long long u = peek(total);
-        while (u == Word<double>::MARK && keepWaiting(polls, limit, ks, fail)) u = peek(total);
+        while (u == Word<double>::MARK && keepWaiting(polls, limit, &ks->stuck, fail)) u = peek(total);
         sh[K * NW + tid] = asValue<double>(u);
     }
     __syncthreads();
@@ -371,7 +263,7 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
                         miss = true;
                         u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
                     }
-            if (!miss || !keepWaiting(polls, rv.spin, ks, &fail)) break;
+            if (!miss || !keepWaiting(polls, rv.spin, &ks->stuck, &fail)) break;
         }
     };
     auto keep = [&](int q, const T (&w)[R]) {

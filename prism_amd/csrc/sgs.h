@@ -40,7 +40,7 @@ struct SgsState {
     int done;           // 1 converged, 3 NaN, 4 b == 0
     int flag;           // 2 rho breakdown: restart with r0 = r = b - A x
     int bad_diag;       // a zero or non-finite diagonal entry
-    int pad;
+    int stuck;          // a wait of the resident kernel ran out
 };
 
 struct SgsView {
@@ -71,6 +71,19 @@ void launch_sgs_scatter(const Launch& L, int n, const int* perm, const double* s
 void launch_sgs_seed(const Launch& L, const SgsView& V, bool start);
 // One iteration k; fresh: 1 right after the start seed, 2 right after a restart seed, else 0.
 void launch_sgs_iteration(const Launch& L, const SgsView& V, long long k, int fresh);
+// Up to R.quota iterations from iteration k in one launch (sgs_resident.hip), for systems of one
+// position per thread on at most n_cu - 1 blocks (sgs_resident_fits; wmax: entries of the widest
+// slice), bit for bit the iterations of launch_sgs_iteration.  pub: 6 n words that start as the
+// mark; line, stale: two sets of resident_sums(blocks) words, swapped after each launch.  When a
+// wait runs out (st->stuck) only x is left in a usable state.
+struct SgsResidentView {
+    double* pub;
+    unsigned long long *line, *stale;
+    int blocks, quota;
+    unsigned spin;
+};
+bool sgs_resident_fits(int n, int wmax, int n_cu, int* blocks);
+void launch_sgs_resident(const Launch& L, const SgsView& V, const SgsResidentView& R, int wmax, long long k, int fresh);
 // ||b - A x||^2 and ||b||^2 partials into part_t (2 G), without touching the iteration's vectors.
 void launch_sgs_true_residual(const Launch& L, const SgsView& V);
 

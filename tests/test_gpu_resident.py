@@ -45,7 +45,7 @@ def solve(hip, A, monkeypatch, resident, **kw):
     x = P.solver.BiCGSTAB(tol=1e-12, max_iters=2000, **kw).step(matrix(hip, A), np.zeros(A.shape[0]), b, out)
     names = set(hip.kernel_stats())
     hip.set_timing(False)
-    return x, b, out[0], any(k.startswith("bicgstab_resident") for k in names)
+    return x, b, out[0], any(k.startswith(("bicgstab_resident", "sgs_resident")) for k in names)
 
 
 SYSTEMS = {
@@ -118,3 +118,26 @@ def test_two_threads_share_the_device(hip, monkeypatch):
     for k in range(2):
         for x in out[k]:
             np.testing.assert_array_equal(x, alone)
+
+
+@pytest.mark.parametrize("n,row", [(1, 1), (64, 3), (257, 4), (513, 5), (5000, 5), (40000, 3)])
+def test_sgs_same_bits_as_its_launches(hip, monkeypatch, n, row):
+    """The resident SGS iteration (sgs_resident.hip), on patterns of two to eight colours."""
+    print(f"case resident sgs {n} {row}", flush=True)
+    offsets = [o for k in range(1, (row + 1) // 2 + 1) for o in (-(7 * k * k - 6), 7 * k * k - 6) if 7 * k * k - 6 < n]
+    A = diagonals(n, tuple(offsets)) if offsets else scattered(1, 1)
+    x1, b, r1, used1 = solve(hip, A, monkeypatch, True, precond="sgs")
+    x0, _, r0, used0 = solve(hip, A, monkeypatch, False, precond="sgs")
+    assert used1 and not used0
+    np.testing.assert_array_equal(x1, x0)
+    assert (r1.krylov_iters, r1.restarts, r1.converged) == (r0.krylov_iters, r0.restarts, r0.converged)
+    assert np.linalg.norm(b - A @ x1) <= 2e-12 * np.linalg.norm(b)
+
+
+def test_sgs_wait_that_runs_out_falls_back(hip, monkeypatch):
+    print("case resident sgs spin", flush=True)
+    monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
+    A = diagonals(5000, (-22, -1, 1, 22))
+    x, b, r, _ = solve(hip, A, monkeypatch, True, precond="sgs")
+    assert r.converged
+    assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
