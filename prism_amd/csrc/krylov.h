@@ -91,13 +91,14 @@ size_t scaled_residual_partials(int64_t n);
 void launch_scaled_residual(const Launch& L, int n, const int* rp, const int* col, const double* val,
                             const int* diag, const double* x, const double* b, double* part, size_t part_cap,
                             KrylovScalars* ks);
-// r64 = b - A64 x64; rr_true (and on start bb, tol2) into ks.
+// r64 = b - A64 x64; rr_true (and on start bb, tol2) into ks.  seed 0, 1, 2 (else -1) seeds the
+// iteration in the same pass: r = T(r64); 1: r0 = r, p = v = 0, rho/alpha/omega = 1; 2: r0 = r
+// (restart); mixed: x32 = 0; leaves the (r,r), (r0,r) partials for the first iteration.
 template <typename T>
-void launch_residual(const Launch& L, const KView<T>& kv, const double* b, const double* x64, double* r64, int start);
-// r = T(r64); start 1: r0 = r, p = v = 0, rho/alpha/omega = 1; start 2: r0 = r (restart);
-// mixed: x32 = 0.  Leaves the (r,r), (r0,r) partials for the first iteration.
-template <typename T>
-void launch_seed(const Launch& L, const KView<T>& kv, const double* r64, int start);
+void launch_residual(const Launch& L, const KView<T>& kv, const double* b, const double* x64, double* r64, int start,
+                     int seed);
+// `bytes` (a multiple of 8) of device memory into pinned host memory, in stream order.
+void launch_read_back(const Launch& L, const void* src, void* dst, size_t bytes);
 template <typename T>
 void launch_iteration(const Launch& L, const KView<T>& kv);
 // Three-kernel iteration (V: alpha, v, s; T: t and four dots; X: omega, rho, beta, x, r, p).

@@ -65,24 +65,6 @@ __device__ inline double waveMax(double v) {
     return v;
 }
 
-// Every block: the K totals of the previous kernel's partials (index order, wavefront 0).
-template <int K>
-__device__ inline void reducePartials(const double* __restrict__ part, int G, double (&out)[K]) {
-    __shared__ double sh[K];
-    if (threadIdx.x < 64) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            double s = 0.0;
-            for (int i = threadIdx.x; i < G; i += 64) s += part[k * G + i];
-            s = waveSum(s);
-            if (threadIdx.x == 0) sh[k] = s;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; ++k) out[k] = sh[k];
-}
-
 // This block's K partial sums into part[k * G + lb].
 template <int K>
 __device__ inline void writePartials(double (&v)[K], double* __restrict__ part, int G, int lb) {
@@ -296,15 +278,27 @@ __device__ inline T sellRow(const int* __restrict__ soff, const int* __restrict_
     case 8: return sellExact<8, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
     default: break;
     }
+    // other widths: eight slots at a time (past the last one, it again), their loads together
     T sum = T(0);
     const T xi = DIFF ? op(row) : T(0);
-    for (int k = 0; k < w; ++k) {
-        const int p = (int)sellPos(o, w, k, lane);
-        int j;
-        if constexpr (REL) j = row + sbase[(o >> 6) + k] + (int)srel[p];
-        else j = scol[p];
-        if (DIFF && j != row) sum += sval[p] * (op(j) - xi);
-        else if (DIFF != 2) sum += sval[p] * op(j);
+    for (int k0 = 0; k0 < w; k0 += 8) {
+        int cj[8];
+        T vv[8], xv[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int k = min(k0 + q, w - 1), p = (int)sellPos(o, w, k, lane);
+            vv[q] = sval[p];
+            if constexpr (REL) cj[q] = row + sbase[(o >> 6) + k] + (int)srel[p];
+            else cj[q] = scol[p];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) xv[q] = op(cj[q]);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (k0 + q >= w) break;
+            if (DIFF && cj[q] != row) sum += vv[q] * (xv[q] - xi);
+            else if (DIFF != 2) sum += vv[q] * xv[q];
+        }
     }
     return sum;
 }
@@ -1209,22 +1203,46 @@ __global__ void k_rhat(int n, const int* cscp, const int* cscr, const int* cscm,
     const double dj = dinv ? dinv[j] : 1.0;
     // the operator's diagonal entry in the difference form (used where i == j)
     auto diagEntry = [&]() {
+        const int q0 = rp[j], q1 = rp[j + 1];
         double rs = 0.0;
-        for (int q = rp[j]; q < rp[j + 1]; ++q) rs += dinv ? val[q] * dinv[col[q]] : val[q];
-        double a = diff == 2 ? 0.0 : (double)(T)rs;  // 2: zero row sums
-        for (int q = rp[j]; q < rp[j + 1]; ++q)
-            if (col[q] != j) a -= (double)(T)(dinv ? val[q] * dinv[col[q]] : val[q]);
+        if (diff != 2)  // 2: zero row sums
+            for (int q8 = q0; q8 < q1; q8 += 8) {
+                double t[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int k = min(q8 + q, q1 - 1);
+                    t[q] = dinv ? val[k] * dinv[col[k]] : val[k];
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    if (q8 + q < q1) rs += t[q];
+            }
+        double a = diff == 2 ? 0.0 : (double)(T)rs;
+        for (int q8 = q0; q8 < q1; q8 += 8) {
+            double t[8];
+            int cq[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int k = min(q8 + q, q1 - 1);
+                cq[q] = col[k];
+                t[q] = (double)(T)(dinv ? val[k] * dinv[cq[q]] : val[k]);
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (q8 + q < q1 && cq[q] != j) a -= t[q];
+        }
         return a;
     };
     const int k0 = cscp[j], k1 = cscp[j + 1];
+    const double dg = diff ? diagEntry() : 0.0;
     double y = 0.0;
-    if (k1 > k0 && k1 - k0 <= 8) {
-        // columns of 1 to 8 entries: every index, value and r0 load issued before the sums
-        // (a slot past the column's end re-reads its last entry and is dropped); same order
+    // eight entries at a time, their index, value and r0 loads issued before the sums (a slot
+    // past the column's end re-reads its last entry and is dropped)
+    for (int k8 = k0; k8 < k1; k8 += 8) {
         int ri[8], mi[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const int k = k0 + q < k1 ? k0 + q : k1 - 1;
+            const int k = min(k8 + q, k1 - 1);
             ri[q] = cscr[k];
             mi[q] = cscm[k];
         }
@@ -1236,16 +1254,9 @@ __global__ void k_rhat(int n, const int* cscp, const int* cscr, const int* cscm,
         }
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            if (k0 + q >= k1) break;
-            const double a = (diff && ri[q] == j) ? diagEntry() : av[q];
+            if (k8 + q >= k1) break;
+            const double a = (diff && ri[q] == j) ? dg : av[q];
             y += a * xv[q];
-        }
-    } else {
-        for (int k = k0; k < k1; ++k) {
-            const int i = cscr[k];
-            double a = (double)(T)(dinv ? val[cscm[k]] * dj : val[cscm[k]]);
-            if (diff && i == j) a = diagEntry();
-            y += a * (double)(T)r0[i];
         }
     }
     rhat[j] = (T)y;
@@ -1264,50 +1275,28 @@ __global__ void k_rowsum_diag(int n, const int* rp, const int* col, const int* d
 }
 
 // ------------------------------------------------------------------ start / events ----
-// r64 = b - A64 x64 (FP64); partials of (r,r), (b,b).
+// r64 = b - A64 x64 (FP64); partials of (r,r), (b,b).  seed >= 0 seeds the iteration in the same
+// pass: r = T(r64); 1 fresh (r0 = r, p = v = 0), 2 restart (r0 = r), 0 residual replacement
+// (r0 kept); mixed precision: x32 = 0; partials (r,r), (r0,r), (r0,r0) in part_seed.
 template <typename T, int FMT>
 __global__ void __launch_bounds__(BS) k_residual(KView<T> kv, const double* b, const double* x64, double* r64,
-                                                 double* part_out) {
+                                                 double* part_out, int seed, double* part_seed) {
     const int lb = logicalBlock(kv.G);
-    double rr = 0.0, bb = 0.0;
+    double v[2] = {0.0, 0.0}, w[3] = {0.0, 0.0, 0.0};
     RowRange R(kv.n, kv.slices_per_block, lb);
     for (int row = R.r0 + threadIdx.x; row < R.r1; row += BS) {
         double ax = matRow<FMT, 0>(kv, kv.sval64, row, [&](int j) { return x64[j]; });
-        double ri = b[row] - ax;
-        r64[row] = ri;
-        rr += ri * ri;
-        bb += b[row] * b[row];
-    }
-    double v[2] = {rr, bb};
-    writePartials<2>(v, part_out, kv.G, lb);
-}
-
-__global__ void k_residual_finish(KrylovScalars* ks, const double* part, int G, int start) {
-    double red[2];
-    reducePartials<2>(part, G, red);
-    if (threadIdx.x == 0) {
-        ks->rr_true = red[0];
-        if (start) {
-            ks->bb = red[1];
-            ks->tol2 = ks->tol * ks->tol * red[1];
-        }
-    }
-}
-
-// r = T(r64); start 1: fresh (r0 = r, p = v = 0); start 2: restart (r0 = r); start 0:
-// residual replacement (r0 kept).  Mixed precision: x32 = 0.  Partials: (r,r), (r0,r), (r0,r0).
-template <typename T>
-__global__ void __launch_bounds__(BS) k_seed(KView<T> kv, const double* r64, int start, double* part_out) {
-    const int lb = logicalBlock(kv.G);
-    double v[3] = {0.0, 0.0, 0.0};
-    RowRange R(kv.n, kv.slices_per_block, lb);
-    for (int row = R.r0 + threadIdx.x; row < R.r1; row += BS) {
-        T ri = (T)r64[row];
+        double r = b[row] - ax;
+        r64[row] = r;
+        v[0] += r * r;
+        v[1] += b[row] * b[row];
+        if (seed < 0) continue;
+        T ri = (T)r;
         kv.r[row] = ri;
         T r0i;
-        if (start) {
+        if (seed) {
             kv.r0[row] = ri;
-            if (start == 1) {
+            if (seed == 1) {
                 kv.p_old[row] = T(0);
                 kv.v_old[row] = T(0);
             }
@@ -1317,11 +1306,46 @@ __global__ void __launch_bounds__(BS) k_seed(KView<T> kv, const double* r64, int
         }
         if (kv.mixed) kv.x[row] = T(0);
         double rd = (double)ri, r0d = (double)r0i;
-        v[0] += rd * rd;
-        v[1] += r0d * rd;
-        v[2] += r0d * r0d;
+        w[0] += rd * rd;
+        w[1] += r0d * rd;
+        w[2] += r0d * r0d;
     }
-    writePartials<3>(v, part_out, kv.G, lb);
+    writePartials<2>(v, part_out, kv.G, lb);
+    if (seed >= 0) writePartials<3>(w, part_seed, kv.G, lb);
+}
+
+// The totals of the residual's (waves 0, 1) and the seed's (waves 2 to 4) partial sums into ks.
+__global__ void __launch_bounds__(320) k_residual_finish(KrylovScalars* ks, const double* part, const double* part_seed,
+                                                         int G, int start, int seed) {
+    __shared__ double sh[5];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (w < 2 || seed >= 0) {
+        const double* p = w < 2 ? part + w * G : part_seed + (w - 2) * G;
+        double s = 0.0;
+#pragma unroll 4
+        for (int i = lane; i < G; i += 64) s += p[i];
+        s = waveSum(s);
+        if (lane == 0) sh[w] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    ks->rr_true = sh[0];
+    if (start) {
+        ks->bb = sh[1];
+        ks->tol2 = ks->tol * ks->tol * sh[1];
+    }
+    if (seed < 0) return;
+    ks->rr = sh[2];
+    if (seed) ks->r0n = sh[4];
+    if (seed == 1) {
+        ks->rho[0] = ks->rho[1] = 1.0;
+        ks->alpha = 1.0;
+        ks->omega = 1.0;
+    }
+    ks->rr_ref = ks->rr_true;
+    ks->flag = 0;
+    if (ks->bb == 0.0) ks->done = 4;
+    else if (ks->rr_true <= ks->tol2) ks->done = 1;
 }
 
 // Clears the event state before a seed: done (clear_done) and the iteration counter (clear_iter).
@@ -1332,22 +1356,10 @@ __global__ void k_reset_events(KrylovScalars* ks, int clear_done, int clear_iter
     }
 }
 
-__global__ void k_seed_finish(KrylovScalars* ks, const double* part, int G, int start) {
-    double red[3];
-    reducePartials<3>(part, G, red);
-    if (threadIdx.x == 0) {
-        ks->rr = red[0];
-        if (start) ks->r0n = red[2];
-        if (start == 1) {
-            ks->rho[0] = ks->rho[1] = 1.0;
-            ks->alpha = 1.0;
-            ks->omega = 1.0;
-        }
-        ks->rr_ref = ks->rr_true;
-        ks->flag = 0;
-        if (ks->bb == 0.0) ks->done = 4;
-        else if (ks->rr_true <= ks->tol2) ks->done = 1;
-    }
+// A few words to pinned host memory, which the host reads after it has waited for the stream: a
+// launch instead of a copy command.
+__global__ void k_read_back(const unsigned long long* src, unsigned long long* dst, int words) {
+    for (int i = threadIdx.x; i < words; i += 64) dst[i] = src[i];
 }
 
 // CSR values -> sliced-ELL values (padding slots stay zero)
@@ -1641,28 +1653,23 @@ inline int formatOf(const KV& kv) {
 }
 
 template <typename T>
-void launch_residual(const Launch& L, const KView<T>& kv, const double* b, const double* x64, double* r64,
-                     int start) {
+void launch_residual(const Launch& L, const KView<T>& kv, const double* b, const double* x64, double* r64, int start,
+                     int seed) {
+    const char* label = seed < 0 ? "bicgstab_residual_f64" : "bicgstab_residual_seed";
     switch (formatOf(kv)) {
     case FMT_DIA:
-        KLAUNCH("bicgstab_residual_f64", (k_residual<T, FMT_DIA>), kv.G, BS, kv, b, x64, r64, kv.part_out);
+        KLAUNCH(label, (k_residual<T, FMT_DIA>), kv.G, BS, kv, b, x64, r64, kv.part_out, seed, kv.part_in);
         break;
     case FMT_DIA_SYM:
-        KLAUNCH("bicgstab_residual_f64", (k_residual<T, FMT_DIA_SYM>), kv.G, BS, kv, b, x64, r64, kv.part_out);
+        KLAUNCH(label, (k_residual<T, FMT_DIA_SYM>), kv.G, BS, kv, b, x64, r64, kv.part_out, seed, kv.part_in);
         break;
     case FMT_SELL16:
-        KLAUNCH("bicgstab_residual_f64", (k_residual<T, FMT_SELL16>), kv.G, BS, kv, b, x64, r64, kv.part_out);
+        KLAUNCH(label, (k_residual<T, FMT_SELL16>), kv.G, BS, kv, b, x64, r64, kv.part_out, seed, kv.part_in);
         break;
     default:
-        KLAUNCH("bicgstab_residual_f64", (k_residual<T, FMT_SELL32>), kv.G, BS, kv, b, x64, r64, kv.part_out);
+        KLAUNCH(label, (k_residual<T, FMT_SELL32>), kv.G, BS, kv, b, x64, r64, kv.part_out, seed, kv.part_in);
     }
-    KLAUNCH("bicgstab_residual_finish", k_residual_finish, 1, 64, kv.ks, kv.part_out, kv.G, start);
-}
-template <typename T>
-void launch_seed(const Launch& L, const KView<T>& kv, const double* r64, int start) {
-    KLAUNCH(sizeof(T) == 8 ? "bicgstab_seed_f64" : "bicgstab_seed_f32", k_seed<T>, kv.G, BS, kv, r64, start,
-            kv.part_in);
-    KLAUNCH("bicgstab_seed_finish", k_seed_finish, 1, 64, kv.ks, kv.part_in, kv.G, start);
+    KLAUNCH("bicgstab_residual_finish", k_residual_finish, 1, 320, kv.ks, kv.part_out, kv.part_in, kv.G, start, seed);
 }
 // part_in: (r,r), (r0,r) of the previous iteration (written back by C); part_out: two
 // scratch partial buffers of 3 x G.
@@ -1801,6 +1808,10 @@ void launch_dia_symcheck(const Launch& L, const KView<double>& kv, const double*
 void launch_reset_events(const Launch& L, KrylovScalars* ks, bool clear_done, bool clear_iter) {
     KLAUNCH("bicgstab_reset_events", k_reset_events, 1, 64, ks, clear_done ? 1 : 0, clear_iter ? 1 : 0);
 }
+void launch_read_back(const Launch& L, const void* src, void* dst, size_t bytes) {
+    KLAUNCH("read_back", k_read_back, 1, 64, static_cast<const unsigned long long*>(src),
+            static_cast<unsigned long long*>(dst), (int)(bytes / 8));
+}
 void launch_flush(const Launch& L, int n, double* x64, float* x32) {
     KLAUNCH("bicgstab_flush", k_flush, nb(n), BS, n, x64, x32);
 }
@@ -1835,10 +1846,10 @@ void launch_to_sell(const Launch& L, int64_t nnz, const int* csr2sell, const dou
     KLAUNCH(sizeof(T) == 8 ? "to_sell_f64" : "to_sell_f32", k_to_sell<T>, nb(nnz), BS, nnz, csr2sell, val, sval);
 }
 
-template void launch_residual<double>(const Launch&, const KView<double>&, const double*, const double*, double*, int);
-template void launch_residual<float>(const Launch&, const KView<float>&, const double*, const double*, double*, int);
-template void launch_seed<double>(const Launch&, const KView<double>&, const double*, int);
-template void launch_seed<float>(const Launch&, const KView<float>&, const double*, int);
+template void launch_residual<double>(const Launch&, const KView<double>&, const double*, const double*, double*, int,
+                                      int);
+template void launch_residual<float>(const Launch&, const KView<float>&, const double*, const double*, double*, int,
+                                     int);
 template void launch_iteration<double>(const Launch&, const KView<double>&);
 template void launch_iteration<float>(const Launch&, const KView<float>&);
 template void launch_rhat<double>(const Launch&, const KView<double>&, const double*, const double*);

@@ -124,7 +124,7 @@ struct prism_ctx {
     std::vector<hipEvent_t> pool;
     std::map<std::string, std::pair<int64_t, double>> stats;
     std::vector<std::string> order;
-    KrylovScalars* hks{nullptr};  // pinned mirror
+    void* hks{nullptr};  // pinned: the scalars last read back (KrylovScalars or SgsState)
     unsigned char* scratch{nullptr};  // this device's static scratch array (scratch_address)
     int n_cu{0};                      // compute units of the device
 
@@ -761,6 +761,7 @@ struct prism_csr {
     int wmax{0};          // entries of the widest sliced-ELL slice
     bool all_diag{true};  // every row stores its diagonal entry
     DevBuf<double> val;
+    DevBuf<double> io[3];  // vectors of the calls on host arrays
     Workspace ws;
     SgsCache sgs;
 };
@@ -967,9 +968,9 @@ hipGraphExec_t iterationPair(Workspace& w, const Launch& L, KView<T>& kv, SetIte
 }
 
 KrylovScalars pollScalars(prism_ctx* ctx, Workspace& w) {
-    HIPCHECK(hipMemcpyAsync(ctx->hks, w.ks.p, sizeof(KrylovScalars), hipMemcpyDeviceToHost, ctx->stream));
+    launch_read_back(ctx->launch(), w.ks.p, ctx->hks, sizeof(KrylovScalars));
     HIPCHECK(hipStreamSynchronize(ctx->stream));
-    return *ctx->hks;
+    return *static_cast<KrylovScalars*>(ctx->hks);
 }
 
 // One BiCGSTAB step x <- BiCGSTAB(A, b, x) (bicgstab.cpp:7-9 semantics: a full solve from the
@@ -1049,10 +1050,9 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     V.part_t = W.part_t.p;
     V.st = W.st.p;
     auto poll = [&] {
-        SgsState s{};
-        HIPCHECK(hipMemcpyAsync(&s, W.st.p, sizeof(s), hipMemcpyDeviceToHost, st));
+        launch_read_back(L, W.st.p, ctx->hks, sizeof(SgsState));
         ctx->sync();
-        return s;
+        return *static_cast<SgsState*>(ctx->hks);
     };
     if (poll().bad_diag) fail(PRISM_ERR_RUNTIME, "SGS preconditioner: a diagonal entry is zero or not finite");
     launch_sgs_seed(L, V, true);
@@ -1067,8 +1067,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
         const size_t words = resident_sums(rv.blocks);
         W.pub.alloc(6 * (size_t)n);
         W.lines.alloc(2 * words);
-        launch_resident_mark<double>(L, W.pub.p, W.pub.n);
-        launch_resident_mark<double>(L, reinterpret_cast<double*>(W.lines.p), W.lines.n);
+        launch_resident_mark<double>(L, W.pub.p, W.pub.n, W.lines.p, W.lines.n);
         rv.pub = W.pub.p;
         rv.line = W.lines.p;
         rv.stale = W.lines.p + words;
@@ -1263,8 +1262,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             const size_t words = resident_sums(plan.blocks);
             pub->alloc(5 * (size_t)A.n);
             w.slots.alloc(2 * words);
-            launch_resident_mark<T>(L, pub->p, pub->n);
-            launch_resident_mark<double>(L, reinterpret_cast<double*>(w.slots.p), w.slots.n);
+            launch_resident_mark<T>(L, pub->p, pub->n, w.slots.p, w.slots.n);
             rv.pub = pub->p;
             rv.slots = w.slots.p;
             rv.stale = w.slots.p + words;
@@ -1272,6 +1270,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             rv.rows = plan.rows;
             rv.quota = RESIDENT_QUOTA;
             rv.spin = residentSpin();
+            rv.x64 = x;
         }
         auto setIter = [&](long long k) {  // buffers and rho slot of iteration k
             int q = (int)(k & 1);
@@ -1291,8 +1290,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             launch_entry<T>(L, kv);
         };
         setIter(0);
-        launch_residual<T>(L, kv, b, x, w.r64.p, 1);
-        launch_seed<T>(L, kv, w.r64.p, 1);
+        launch_residual<T>(L, kv, b, x, w.r64.p, 1, 1);
         enter(1);
         // FP32 refinement guard.  The three-kernel form takes alpha from (rhat, p) and rho
         // from (r0, s) - omega (r0, t); in FP32 these part from the stored v and r by
@@ -1312,10 +1310,9 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             if (traceEnabled()) std::fprintf(stderr, "krylov n=%d: FP32 divergence at iteration %lld\n", A.n, nit);
             HIPCHECK(hipMemcpyAsync(x, w.xsave.p, A.n * sizeof(double), hipMemcpyDeviceToDevice, st));
             if (retries++ == 0) {
-                launch_residual<T>(L, kv, b, x, w.r64.p, 0);
                 launch_reset_events(L, w.ks.p, true, false);
                 setIter(nit);
-                launch_seed<T>(L, kv, w.r64.p, 1);
+                launch_residual<T>(L, kv, b, x, w.r64.p, 0, 1);
                 enter(1);
                 ++out.refinements;
                 return true;
@@ -1340,18 +1337,20 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         long long best_iter = 0;
         double last_true = INFINITY;
         bool forced = false;  // the pending reliable update was forced by stagnation
+        bool resident_last = false;  // the launch before this poll was the resident kernel
         int stalls = 0;       // forced updates in a row that did not lower the FP64 residual
         for (;;) {
             KrylovScalars s = pollScalars(ctx, w);
             ticket.give();
+            const bool flushed = resident_last && s.flag;  // by the resident kernel
+            resident_last = false;
             if (s.stuck) {  // a wait of the resident kernel ran out: on from this x without it
                 if (traceEnabled()) std::fprintf(stderr, "krylov n=%d: resident kernel stuck\n", A.n);
                 plan.blocks = 0;
                 if constexpr (sizeof(T) == 4) launch_flush(L, A.n, x, kv.x);
-                launch_residual<T>(L, kv, b, x, w.r64.p, 0);
                 launch_reset_events(L, w.ks.p, true, false);
                 setIter(s.nit);
-                launch_seed<T>(L, kv, w.r64.p, 1);
+                launch_residual<T>(L, kv, b, x, w.r64.p, 0, 1);
                 enter(1);
                 continue;
             }
@@ -1380,31 +1379,30 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             }
             setIter(s.nit);
             if (s.flag == 2) {  // rho breakdown: Eigen restarts with r0 = r = b - A x (keeps p, v)
-                if constexpr (sizeof(T) == 4) launch_flush(L, A.n, x, kv.x);
-                launch_residual<T>(L, kv, b, x, w.r64.p, 0);
-                launch_seed<T>(L, kv, w.r64.p, 2);
+                if constexpr (sizeof(T) == 4)
+                    if (!flushed) launch_flush(L, A.n, x, kv.x);
+                launch_residual<T>(L, kv, b, x, w.r64.p, 0, 2);
                 if (out.restarts++ == 0) launch_reset_events(L, w.ks.p, false, true);
                 enter(2);
                 ++out.refinements;
                 continue;
             }
             if (s.flag == 1) {  // mixed: reliable update of x and r in FP64
-                if constexpr (sizeof(T) == 4) launch_flush(L, A.n, x, kv.x);
-                launch_residual<T>(L, kv, b, x, w.r64.p, 0);
-                if (have_xsave) {
-                    KrylovScalars u = pollScalars(ctx, w);
-                    if (!(u.rr_true == u.rr_true) || u.rr_true > 1e4 * last_true) {
+                if constexpr (sizeof(T) == 4)
+                    if (!flushed) launch_flush(L, A.n, x, kv.x);
+                const int start = refineRestart(symmetric) ? 1 : 0;
+                launch_residual<T>(L, kv, b, x, w.r64.p, 0, start);
+                enter(start);
+                KrylovScalars t = pollScalars(ctx, w);
+                if (have_xsave) {  // a divergence drops this seed (diverged() seeds again)
+                    if (!(t.rr_true == t.rr_true) || t.rr_true > 1e4 * last_true) {
                         if (diverged(s.nit)) continue;
                         break;
                     }
-                    if (u.rr_true <= last_true)
+                    if (t.rr_true <= last_true)
                         HIPCHECK(hipMemcpyAsync(w.xsave.p, x, A.n * sizeof(double), hipMemcpyDeviceToDevice, st));
                 }
-                const int start = refineRestart(symmetric) ? 1 : 0;
-                launch_seed<T>(L, kv, w.r64.p, start);
-                enter(start);
                 ++out.refinements;
-                KrylovScalars t = pollScalars(ctx, w);
                 if (t.done) { out.done = t.done; out.iters = t.nit; break; }
                 if (t.iter >= t.maxit) { out.done = 2; out.iters = t.nit; break; }
                 if (forced) {  // two stalled windows in a row that the update did not help:
@@ -1442,6 +1440,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             last_rr = s.rr;
             if (plan.blocks > 0 && ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu)) {
                 launch_resident<T>(L, kv, rv, plan);
+                resident_last = true;
                 std::swap(rv.slots, rv.stale);
             } else if (three) {
                 for (int k = 0; k < chunk; ++k) {
@@ -1459,7 +1458,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             }
         }
         // true relative residual ||b - A x|| / ||b|| (FP64)
-        launch_residual<T>(L, kv, b, x, w.r64.p, 0);
+        launch_residual<T>(L, kv, b, x, w.r64.p, 0, -1);
         KrylovScalars f = pollScalars(ctx, w);
         out.rel = f.bb > 0 ? std::sqrt(f.rr_true / f.bb) : 0.0;
         if (traceEnabled())
@@ -1687,7 +1686,8 @@ API int prism_ctx_create(int device, prism_ctx** out) {
         auto c = std::make_unique<prism_ctx>();
         c->device = device;
         HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-        HIPCHECK(hipHostMalloc((void**)&c->hks, sizeof(KrylovScalars), hipHostMallocDefault));
+        static_assert(sizeof(KrylovScalars) % 8 == 0 && sizeof(SgsState) % 8 == 0);
+        HIPCHECK(hipHostMalloc(&c->hks, std::max(sizeof(KrylovScalars), sizeof(SgsState)), hipHostMallocDefault));
         c->scratch = static_cast<unsigned char*>(scratch_address(device));
         HIPCHECK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device));
         *out = c.release();
@@ -2289,7 +2289,7 @@ API int prism_csr_create(prism_ctx* ctx, int64_t n, const int64_t* rp, const int
 API int prism_csr_destroy(prism_csr* a) { return guard([&] { delete a; }); }
 API int prism_csr_spmv(prism_csr* a, const double* x, double* y) {
     return guard([&] {
-        DevBuf<double> dx, dy;
+        DevBuf<double>&dx = a->io[0], &dy = a->io[1];
         dx.upload(x, a->n, a->ctx->stream);
         dy.alloc(a->n);
         launch_spmv64(a->ctx->launch(), (int)a->n, a->rp.p, a->col.p, a->val.p, dx.p, dy.p);
@@ -2299,7 +2299,7 @@ API int prism_csr_spmv(prism_csr* a, const double* x, double* y) {
 }
 API int prism_csr_jacobi_step(prism_csr* a, const double* b, const double* xin, double* xout) {
     return guard([&] {  // jacobi.cpp:5-9: x + D^-1 (b - A x), on the device
-        DevBuf<double> db, dx, dy;
+        DevBuf<double>&db = a->io[0], &dx = a->io[1], &dy = a->io[2];
         db.upload(b, a->n, a->ctx->stream);
         dx.upload(xin, a->n, a->ctx->stream);
         dy.alloc(a->n);
@@ -2312,7 +2312,7 @@ API int prism_csr_bicgstab(prism_csr* a, const double* b, const double* xin, dou
                            const prism_solve_params* p, prism_solve_result* r) {
     return guard([&] {
         if (!a || !p || !b || !xin || !xout) fail(PRISM_ERR_INVALID, "BiCGSTAB::step: null argument");
-        DevBuf<double> db, dx;
+        DevBuf<double>&db = a->io[0], &dx = a->io[1];
         db.upload(b, a->n, a->ctx->stream);
         dx.upload(xin, a->n, a->ctx->stream);
         MatRef A{(int)a->n, a->rp.p, a->col.p, a->diag.p, a->val.p, (int64_t)a->val.n,

@@ -32,14 +32,15 @@ struct ResidentView {
     int blocks, rows;
     int quota;                  // iterations of this launch at most
     unsigned spin;              // polls of one wait at most
+    double* x64;                // mixed precision: x is added here (and cleared) when the launch ends on a flag
 };
 
 // Plan for an n-row system (wmax: the longest stored row) on a device of n_cu compute units.
 template <typename T>
 ResidentPlan resident_plan(int64_t n, bool dia, int wmax, int n_cu);
-// Marks `count` words as unwritten.
+// Marks `count` words at p and `more` words at q as unwritten.
 template <typename T>
-void launch_resident_mark(const Launch& L, T* p, size_t count);
+void launch_resident_mark(const Launch& L, T* p, size_t count, unsigned long long* q, size_t more);
 // Up to rv.quota iterations from the state in kv (p_new, r, r0, rhat, x and kv.ks, as the
 // three-kernel iteration keeps them) and back into it, to the next event at most.  A wait
 // that runs out (the blocks were not resident together) sets ks->stuck and ends the launch

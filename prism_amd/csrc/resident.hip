@@ -384,12 +384,21 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
     T* pk = even ? kv.p_new : kv.p_old;
     T* pl = even ? kv.p_old : kv.p_new;
     T* vl = even ? kv.v_old : kv.v_new;
+    const bool flush = mixed && flag;
+    if (m > 0 || flush) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int row = rowOf(j);
+            if (row >= r1) continue;
+            if (flush) rv.x64[row] += (double)x[j];
+            kv.x[row] = flush ? T(0) : x[j];
+        }
+    }
     if (m > 0) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             const int row = rowOf(j);
             if (row >= r1) continue;
-            kv.x[row] = x[j];
             kv.r[row] = r[j];
             pk[row] = p[j];
             pl[row] = asValue<T>(bufPeek<U>(pub, rowAt(j), pm_old * bytes));
@@ -425,10 +434,10 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
 }
 
 template <typename T>
-__global__ void k_mark(T* p, size_t count) {
-    using U = typename Word<T>::U;
+__global__ void k_mark(T* p, size_t count, unsigned long long* q, size_t more) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) reinterpret_cast<U*>(p)[i] = Word<T>::MARK;
+    if (i < count) reinterpret_cast<typename Word<T>::U*>(p)[i] = Word<T>::MARK;
+    if (i < more) q[i] = Word<double>::MARK;
 }
 
 template <typename T, bool DIA, int W, int R>
@@ -478,8 +487,9 @@ ResidentPlan resident_plan(int64_t n, bool dia, int wmax, int n_cu) {
 }
 
 template <typename T>
-void launch_resident_mark(const Launch& L, T* p, size_t count) {
-    if (count) PRISM_LAUNCH("resident_mark", k_mark<T>, (int)((count + 255) / 256), 256, p, count);
+void launch_resident_mark(const Launch& L, T* p, size_t count, unsigned long long* q, size_t more) {
+    const size_t most = std::max(count, more);
+    PRISM_LAUNCH("resident_mark", k_mark<T>, (int)((most + 255) / 256), 256, p, count, q, more);
 }
 
 template <typename T>
@@ -497,8 +507,8 @@ void launch_resident(const Launch& L, const KView<T>& kv, const ResidentView<T>&
 
 template ResidentPlan resident_plan<double>(int64_t, bool, int, int);
 template ResidentPlan resident_plan<float>(int64_t, bool, int, int);
-template void launch_resident_mark<double>(const Launch&, double*, size_t);
-template void launch_resident_mark<float>(const Launch&, float*, size_t);
+template void launch_resident_mark<double>(const Launch&, double*, size_t, unsigned long long*, size_t);
+template void launch_resident_mark<float>(const Launch&, float*, size_t, unsigned long long*, size_t);
 template void launch_resident<double>(const Launch&, const KView<double>&, const ResidentView<double>&,
                                       const ResidentPlan&);
 template void launch_resident<float>(const Launch&, const KView<float>&, const ResidentView<float>&,
