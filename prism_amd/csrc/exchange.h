@@ -49,13 +49,13 @@ __device__ inline void post(U* p, U v) {
 constexpr unsigned FAR = 0x80000000u;
 constexpr int AGENT = 16;
 using U2 = unsigned int __attribute__((ext_vector_type(2)));
-template <typename U>
+template <typename U, int POLICY = AGENT>
 __device__ inline U bufPeek(__amdgpu_buffer_rsrc_t b, unsigned at, unsigned base) {
     if constexpr (sizeof(U) == 8) {
-        const U2 v = __builtin_amdgcn_raw_buffer_load_b64(b, at, base, AGENT);
+        const U2 v = __builtin_amdgcn_raw_buffer_load_b64(b, at, base, POLICY);
         return (unsigned long long)v.y << 32 | v.x;
     } else {
-        return __builtin_amdgcn_raw_buffer_load_b32(b, at, base, AGENT);
+        return __builtin_amdgcn_raw_buffer_load_b32(b, at, base, POLICY);
     }
 }
 template <typename U>

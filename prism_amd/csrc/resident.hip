@@ -5,10 +5,10 @@
 // iteration, where the data would take 1-4 us (64^3 cells, 20 MB).  Here one launch runs up
 // to `quota` iterations of the same recurrences.  Each thread keeps R rows: their matrix entries
 // (values and element addresses) and their elements of x, r, r0, rhat, p, v, s and t stay in
-// registers from the first iteration to the last, so an iteration moves only p and s between
-// blocks, and the partial sums of its two reductions.  Per iteration, three kernels -> this
+// registers from the first iteration to the last (but see keptRows), so an iteration moves only
+// p and s between blocks, and the partial sums of its two reductions.  Per iteration, three kernels -> this
 // one: 200 rows FP64 14 -> 2.6 us, 16,384 rows FP64 15 -> 5.8 us, 82,944 rows of tetrahedra
-// FP32 17.5 -> 7.4 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us.  What
+// FP32 17.5 -> 7.4 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us, 512,000 rows FP64 29.8 -> 18.7 us.  What
 // bounds it now is latency: four to five hops of 0.3-0.5 us between blocks per iteration, and
 // at two and three rows per thread the issue of the products (0.7 us per row and product).
 //
@@ -136,12 +136,26 @@ __device__ inline bool awaitTotals(unsigned long long* slot, int G, int lb, unsi
     return *fail == 0;
 }
 
+// Rows per thread up to which the coefficients stay in registers with everything else, and up
+// to which the element addresses do.  Above the first, DIA coefficients (7 per row at most) are
+// read again for each product: a thread's 256 registers hold 9 vectors, addresses and the elements
+// on their way, and the coefficients of the whole system come from the L2s (4 MB each) and the
+// Infinity Cache.  Above the second, the product goes row by row, the next row's elements and
+// coefficients on their way, and forms the addresses each time (the compiler spills 51
+// registers otherwise).  Per iteration, all rows at once / row by row: FP64 4 rows 18.7 / 21.3 us,
+// 5 rows 30.1 / 26.7 us; FP32 5 rows 16.9 / 17.6 us, 6 rows 18.6 / 22.2 us, 7 rows 27.4 / 25.8 us.
+template <typename T>
+constexpr int keptRows() { return sizeof(T) == 8 ? 3 : 4; }
+template <typename T>
+constexpr int heldRows() { return sizeof(T) == 8 ? 4 : 6; }
+
 // FP64: plain row products; FP32: the difference form (matRow in krylov.hip; the diagonal
 // coefficient holds the row sum, or zero where the matrix has zero row sums).
 template <typename T, bool DIA, int W, int R>
 __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv) {
     using U = typename Word<T>::U;
     constexpr U MARK = Word<T>::MARK;
+    constexpr bool STREAM = R > keptRows<T>(), BYROW = R > heldRows<T>();
     constexpr bool DIFF = sizeof(T) == 4;
     __shared__ T own[2][R * BS + 1];  // this block's p and s, and a zero
     __shared__ double shA[2 * NW + 2], shC[4 * NW + 4];
@@ -162,8 +176,8 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
 
     // this thread's rows r0 + tid + j BS; at[j][k]: where entry k's element is, as a byte offset
     // into own[] (this block's), or FAR + its byte offset in the published vector
-    T a[R][W], x[R], r[R], z[R], h[R], p[R], v[R], s[R], t[R];
-    unsigned at[R][W];
+    T a[STREAM ? 1 : R][W], x[R], r[R], z[R], h[R], p[R], v[R], s[R], t[R];
+    unsigned at[BYROW ? 1 : R][W];
     auto rowOf = [&](int j) { return r0 + tid + j * BS; };
     auto mine = [&](int j) { return (unsigned)(tid + j * BS) * (unsigned)sizeof(T); };
     auto rowAt = [&](int j) { return rowOf(j) < r1 ? (unsigned)rowOf(j) * (unsigned)sizeof(T) : FAR; };
@@ -189,7 +203,7 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
             if constexpr (DIA) {
                 if (ok && k < kv.ndia && (unsigned)(row + kv.doff[k]) < (unsigned)n) {
                     c = row + kv.doff[k];
-                    e = kv.sval[(int64_t)k * n + row];
+                    if constexpr (!STREAM) e = kv.sval[(int64_t)k * n + row];
                 }
             } else if (k < w) {
                 const int q = (int)sellPos(o, w, k, row & 63);
@@ -197,21 +211,42 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
                 e = kv.sval[q];
             }
             if (DIFF && kv.diff == 2 && c == row) e = T(0);
-            a[j][k] = e;
+            if constexpr (BYROW) continue;
+            if constexpr (!STREAM) a[j][k] = e;
             const int l = ok ? c - r0 : 0;
             at[j][k] = (unsigned)l < (unsigned)rv.rows ? (unsigned)l * (unsigned)sizeof(T)
                                                         : FAR + (unsigned)c * (unsigned)sizeof(T);
         }
     }
+    auto place = [&](int j, int k) {
+        if constexpr (BYROW) {  // formed each time
+            const int l = tid + j * BS + kv.doff[k], c = r0 + l;
+            const bool in = k < kv.ndia && rowOf(j) < r1 && (unsigned)c < (unsigned)n;
+            return !in ? mine(j) : (unsigned)l < (unsigned)rv.rows ? (unsigned)l * (unsigned)sizeof(T)
+                                                                   : FAR + (unsigned)c * (unsigned)sizeof(T);
+        } else {
+            return at[j][k];
+        }
+    };
     unsigned long long wants = 0;  // bit j W + k: some lane of the wave reads entry k of row j from another block
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
         for (int k = 0; k < W; ++k)
-            if (__ballot(at[j][k] >= FAR)) wants |= 1ull << (j * W + k);
+            if (__ballot(place(j, k) >= FAR)) wants |= 1ull << (j * W + k);
     const __amdgpu_buffer_rsrc_t pub =
         __builtin_amdgcn_make_buffer_rsrc(rv.pub, 0, 5 * n * (int)sizeof(T), 0x00020000);
     const unsigned bytes = (unsigned)n * (unsigned)sizeof(T);  // of one published vector
+    const __amdgpu_buffer_rsrc_t vals = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T*>(kv.sval), 0, STREAM ? kv.ndia * n * (int)sizeof(T) : 0, 0x00020000);
+    auto coef = [&](int j, int k) {
+        if constexpr (STREAM) {  // of a row there is none of: reads as zero
+            if (k >= kv.ndia || (DIFF && kv.diff == 2 && kv.doff[k] == 0)) return T(0);
+            return asValue<T>(bufPeek<U, 0>(vals, rowAt(j), (unsigned)k * bytes));
+        } else {
+            return a[j][k];
+        }
+    };
     const bool mixed = kv.mixed != 0, pc = kv.precond != 0;
     const double tol2 = ks->tol2, ref2 = ks->delta2 * ks->rr_ref, tiny = ks->breakdown * ks->r0n;
     double rho = ks->rho[kv.par], alpha = ks->alpha, omega = ks->omega;
@@ -225,45 +260,91 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
     // are the elements looked at one by one.
     auto product = [&](unsigned base, int q, const T (&w)[R], T (&y)[R]) {
         const char* mem = reinterpret_cast<const char*>(own[q]);
-        U u[R][W];
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-#pragma unroll
-            for (int k = 0; k < W; ++k) {
-                asm volatile("" : "+v"(at[j][k]));  // no copies of what follows kept per iteration
-                u[j][k] = U(0);
-                if (wants >> (j * W + k) & 1) u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
-            }
-        unsigned polls = 0;
-        for (;;) {
-            bool nan = false;
-#pragma unroll
-            for (int j = 0; j < R; ++j) {
-                if (j >= live) continue;
-                T sum = T(0);
+        if constexpr (BYROW) {
+            // row by row, with the next row's values, addresses and far elements on their way
+            T cf[2][W];
+            U u[2][W];
+            unsigned pl[2][W];
+            auto issue = [&](int j) {
+                if (j >= live) return;
 #pragma unroll
                 for (int k = 0; k < W; ++k) {
-                    // one of the two is zero: own[q] ends with one, the buffer read was out of range
-                    const U l = asWord(*reinterpret_cast<const T*>(mem + min(at[j][k], (unsigned)(R * BS * sizeof(T)))));
-                    const T e = asValue<T>(l | u[j][k]);
-                    if (DIFF) sum += a[j][k] * (at[j][k] == mine(j) ? w[j] : e - w[j]);
-                    else sum += a[j][k] * e;
+                    pl[j & 1][k] = place(j, k);
+                    cf[j & 1][k] = coef(j, k);
+                    u[j & 1][k] = U(0);
+                    if (wants >> (j * W + k) & 1) u[j & 1][k] = bufPeek<U>(pub, pl[j & 1][k] ^ FAR, base);
                 }
-                y[j] = sum;
-                nan |= sum != sum;
+            };
+            issue(0);
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                if (j + 1 < R) issue(j + 1);
+                if (j >= live) continue;
+                unsigned polls = 0;
+                for (;;) {
+                    T sum = T(0);
+#pragma unroll
+                    for (int k = 0; k < W; ++k) {
+                        const unsigned at = pl[j & 1][k];
+                        const U l = asWord(*reinterpret_cast<const T*>(mem + min(at, (unsigned)(R * BS * sizeof(T)))));
+                        const T e = asValue<T>(l | u[j & 1][k]);
+                        if (DIFF) sum += cf[j & 1][k] * (at == mine(j) ? w[j] : e - w[j]);
+                        else sum += cf[j & 1][k] * e;
+                    }
+                    y[j] = sum;
+                    if (sum == sum) break;
+                    bool miss = false;
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int k = 0; k < W; ++k)
+                        if (u[j & 1][k] == MARK) {
+                            miss = true;
+                            u[j & 1][k] = bufPeek<U>(pub, pl[j & 1][k] ^ FAR, base);
+                        }
+                    if (!miss || !keepWaiting(polls, rv.spin, &ks->stuck, &fail)) break;
+                }
             }
-            if (!nan) break;
-            bool miss = false;
-            asm volatile("" ::: "memory");
+        } else {
+            U u[R][W];
 #pragma unroll
             for (int j = 0; j < R; ++j)
 #pragma unroll
-                for (int k = 0; k < W; ++k)
-                    if (u[j][k] == MARK) {
-                        miss = true;
-                        u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
+                for (int k = 0; k < W; ++k) {
+                    asm volatile("" : "+v"(at[j][k]));  // no copies of what follows kept per iteration
+                    u[j][k] = U(0);
+                    if (wants >> (j * W + k) & 1) u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
+                }
+            unsigned polls = 0;
+            for (;;) {
+                bool nan = false;
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    if (j >= live) continue;
+                    T sum = T(0);
+#pragma unroll
+                    for (int k = 0; k < W; ++k) {
+                        // one of the two is zero: own[q] ends with one, the buffer read was out of range
+                        const U l = asWord(*reinterpret_cast<const T*>(mem + min(at[j][k], (unsigned)(R * BS * sizeof(T)))));
+                        const T e = asValue<T>(l | u[j][k]), c = coef(j, k);
+                        if (DIFF) sum += c * (at[j][k] == mine(j) ? w[j] : e - w[j]);
+                        else sum += c * e;
                     }
-            if (!miss || !keepWaiting(polls, rv.spin, &ks->stuck, &fail)) break;
+                    y[j] = sum;
+                    nan |= sum != sum;
+                }
+                if (!nan) break;
+                bool miss = false;
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < R; ++j)
+#pragma unroll
+                    for (int k = 0; k < W; ++k)
+                        if (u[j][k] == MARK) {
+                            miss = true;
+                            u[j][k] = bufPeek<U>(pub, at[j][k] ^ FAR, base);
+                        }
+                if (!miss || !keepWaiting(polls, rv.spin, &ks->stuck, &fail)) break;
+            }
         }
     };
     auto keep = [&](int q, const T (&w)[R]) {
@@ -307,8 +388,7 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
             if (G > 1) mark(sBase(m - 1));
             markSums(slotA(m - 1), 2);
         }
-        T vn[R] = {};
-        if (live) product(pm * bytes, 0, p, vn);
+        if (live) product(pm * bytes, 0, p, s);  // v_k; v keeps v_{k-1} until the event test
         double red[2];
         if (!awaitTotals<2>(slotA(m), G, lb, rv.spin, ks, shA, &fail, red)) return;
         rp = red[0];
@@ -330,7 +410,7 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
 #pragma unroll
         for (int j = 0; j < R; ++j) {
             if (j >= live) continue;
-            v[j] = vn[j];
+            v[j] = s[j];
             s[j] = r[j] - al * v[j];
         }
         if (G > 1) publish(sBase(m), s);
@@ -449,12 +529,18 @@ void launchOne(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv) {
 template <typename T, bool DIA, int W>
 void launchR(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, int R) {
     switch (R) {
-    case 1: launchOne<T, DIA, W, 1>(L, kv, rv); break;
-    case 2: launchOne<T, DIA, W, 2>(L, kv, rv); break;
-    case 3: launchOne<T, DIA, W, 3>(L, kv, rv); break;
+    case 1: launchOne<T, DIA, W, 1>(L, kv, rv); return;
+    case 2: launchOne<T, DIA, W, 2>(L, kv, rv); return;
+    case 3: launchOne<T, DIA, W, 3>(L, kv, rv); return;
     case 4:
-        if constexpr (sizeof(T) == 4) launchOne<T, DIA, W, 4>(L, kv, rv);
-        break;
+        if constexpr (sizeof(T) == 4 || (DIA && W <= 7)) launchOne<T, DIA, W, 4>(L, kv, rv);
+        return;
+    case 5:
+        if constexpr (DIA && W <= 7) launchOne<T, DIA, W, 5>(L, kv, rv);
+        return;
+    case 6:
+        if constexpr (DIA && W <= 7 && sizeof(T) == 4) launchOne<T, DIA, W, 6>(L, kv, rv);
+        return;
     default: throw Error(PRISM_ERR_RUNTIME, "resident BiCGSTAB: no kernel for this many rows per thread");
     }
 }
@@ -465,14 +551,18 @@ void launchR(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, int
 // block sums).  With one row per thread, the rows per block of the three-kernel iteration: the
 // sums are then formed in the same order, and the iterates are the same bits.  With more, as
 // many blocks as there can be, so that the rows of a block, and with them an iteration's
-// work, are fewest.
+// work, are fewest.  Where the line lies: with up to seven diagonals, FP64 5 rows per thread
+// (652,800 in all) 27.6 us per iteration against 31.9 us of the three kernels at 643,280 rows
+// (its 87 spilled registers leave no room for a sixth); FP32 6 rows (783,360 in all) 18.6 us against 32.8 us (row per thread) at
+// 665,280, while 7 take 25.8 us against 24.9 us of the packed kernels at 847,872.  Else as many
+// as hold their coefficients in registers (keptRows), one with up to 16 entries per row.
 template <typename T>
 ResidentPlan resident_plan(int64_t n, bool dia, int wmax, int n_cu) {
     ResidentPlan p;
     const int W = wmax <= 5 ? 5 : wmax <= 8 ? (dia && wmax <= 7 ? 7 : 8) : wmax <= 16 && !dia ? 16 : 0;
     const int most = std::min(n_cu - 1, RES_MAX_BLOCKS);
     if (!W || n < 1 || most < 1) return p;
-    const int rmax = W == 16 ? 1 : sizeof(T) == 4 ? 4 : 3;
+    const int rmax = W == 16 ? 1 : dia && W <= 7 ? (sizeof(T) == 4 ? 6 : 5) : keptRows<T>();
     int spb = 0;
     krylov_grid(n, &spb);
     int64_t rows = (int64_t)spb * 64;

@@ -83,6 +83,39 @@ def test_several_rows_per_thread(hip, monkeypatch, n, precision):
     assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("n,offsets,precision", [
+    (255 * 1536 + 1, (-4096, -64, -1, 1, 64, 4096), "fp64"), (255 * 2048, (-511, -1, 1, 511), "fp64"),
+    (255 * 2048 + 1, (-4096, -64, -1, 1, 64, 4096), "fp64"), (255 * 2560, (-4097, -63, -1, 1, 63, 4097), "fp64"),
+    (255 * 2560, (-300001, -5, 5, 300001), "fp64"),
+    (255 * 2048 + 1, (-4096, -64, -1, 1, 64, 4096), "fp32"), (255 * 2560 + 1, (-511, -1, 1, 511), "fp32"),
+    (255 * 3072, (-4097, -63, -1, 1, 63, 4097), "fp32")])
+def test_streamed_coefficients(hip, monkeypatch, n, offsets, precision):
+    """Rows per thread at which the coefficients are read again for each product."""
+    print(f"case resident streamed {n} {len(offsets) + 1} {precision}", flush=True)
+    A = diagonals(n, offsets)
+    x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision)
+    assert used
+    assert r.krylov_rel_residual <= 1e-12
+    assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n", [255 * 2048 + 1, 255 * 2560 + 1])
+def test_streamed_zero_row_sums(hip, monkeypatch, n):
+    """FP32 without a diagonal term in the difference form (symmetric, singular, consistent)."""
+    print(f"case resident zero row sums {n}", flush=True)
+    rng = np.random.default_rng(6)
+    U = sp.diags([-rng.integers(32, 64, n - o) / 64.0 for o in (1, 64, 4096)], (1, 64, 4096), shape=(n, n))
+    A = (U + U.T).tocsr()
+    A = (A - sp.diags(np.asarray(A.sum(axis=1)).ravel())).tocsr()
+    A.sort_indices()
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "1")
+    b = A @ rng.standard_normal(n)
+    out = []
+    x = P.solver.BiCGSTAB(tol=1e-10, max_iters=4000, precision="fp32").step(matrix(hip, A), np.zeros(n), b, out)
+    assert out[0].krylov_rel_residual <= 1e-10
+    assert np.linalg.norm(b - A @ x) <= 2e-10 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_wait_that_runs_out_falls_back(hip, monkeypatch, precision):
     """One poll per wait: the blocks give up at their first wait, and the solve goes on with the
