@@ -458,6 +458,15 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
         pm = pm == 2 ? 0 : pm + 1;
     }
 
+    // The totals say that every block has posted its sums, not that it has read its neighbours' p_k
+    // yet: one more round (the next four sums' words are free), after which p_k can be marked, and
+    // no block can give up any more when the first one writes the state.
+    if (G > 1) {
+        const double none[2] = {0.0, 0.0};
+        double all[2];
+        postSums<2>(none, slotC(m), G, lb, shC);
+        if (!awaitTotals<2>(slotC(m), G, lb, rv.spin, ks, shC, &fail, all)) return;
+    }
     // the state as the three-kernel iteration keeps it: p_k and rho_k in slot k & 1, p_{k-1},
     // v_{k-1} and rho_{k-1} in the other one
     const bool even = (m & 1) == 0;

@@ -72,6 +72,17 @@ def test_same_bits_as_three_kernels(hip, monkeypatch, name, precision, precond):
     assert np.linalg.norm(b - A @ x1) <= 2e-12 * np.linalg.norm(b)
 
 
+@pytest.mark.parametrize("n", [6400, 100000])
+def test_ends_of_launches(hip, monkeypatch, n):
+    """Short solves end while blocks may still wait for the last p of others: every one of many
+    has the same bits."""
+    print(f"case resident ends {n}", flush=True)
+    A = scattered(n, 12)
+    x0 = solve(hip, A, monkeypatch, False)[0]
+    for _ in range(20):
+        np.testing.assert_array_equal(solve(hip, A, monkeypatch, True)[0], x0)
+
+
 @pytest.mark.parametrize("n,precision", [(255 * 512 + 1, "fp64"), (262144, "fp64"), (255 * 1536, "fp64"),
                                          (255 * 512 + 1, "fp32"), (400001, "fp32"), (255 * 2048, "fp32")])
 def test_several_rows_per_thread(hip, monkeypatch, n, precision):
