@@ -8,9 +8,10 @@
 // registers from the first iteration to the last (but see keptRows), so an iteration moves only
 // p and s between blocks, and the partial sums of its two reductions.  Per iteration, three kernels -> this
 // one: 200 rows FP64 14 -> 2.6 us, 16,384 rows FP64 15 -> 5.8 us, 82,944 rows of tetrahedra
-// FP32 17.5 -> 7.4 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us, 512,000 rows FP64 29.8 -> 18.7 us.  What
-// bounds it now is latency: four to five hops of 0.3-0.5 us between blocks per iteration, and
-// at two and three rows per thread the issue of the products (0.7 us per row and product).
+// FP32 17.5 -> 7.0 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us,
+// 512,000 rows FP64 29.8 -> 18.7 us.  What bounds it now is latency: four to five hops of
+// 0.3-0.5 us between blocks per iteration, and at two and three rows per thread the products'
+// wait for their neighbours' words (0.7 us per row and product).
 //
 // Exchange without barriers.  A word that another block waits for carries its own flag: it
 // holds the mark, a signalling NaN that no arithmetic produces (results are quiet NaNs), until
@@ -25,7 +26,8 @@
 //   X: omega, beta, x, r, p_{k+1}
 // A block that has T's totals knows that every block has read s_k, the first two totals and
 // p_k: at the start of iteration k + 1 it marks its words of p_{k-1} and s_k and those sums
-// again (p_k stays: an event in iteration k + 1 hands it back to the host's state); T's sums
+// again (p_k stays: an event in iteration k + 1 hands it back to the host's state; the launch's
+// last p is marked after one more round, when every block has read it); T's sums
 // are marked after the next first totals.  Every word marked again is next polled after a
 // reduction that its owner took part in only when the marks were in memory (the s_waitcnt
 // before T's sums), so no reader sees an old value: p has three buffers, s, the sums and the
