@@ -900,7 +900,13 @@ unsigned residentSpin() {
     return e && std::atol(e) > 0 ? (unsigned)std::atol(e) : 1u << 20;
 }
 
-constexpr int RESIDENT_QUOTA = 128;  // iterations of one resident launch
+// Iterations of one resident launch at most (PRISM_KRYLOV_QUOTA: fewer, read per solve).
+constexpr int RESIDENT_QUOTA = 128;
+int residentQuota() {
+    const char* e = std::getenv("PRISM_KRYLOV_QUOTA");
+    const int q = e ? std::atoi(e) : 0;
+    return q > 0 ? std::min(q, RESIDENT_QUOTA) : RESIDENT_QUOTA;
+}
 
 // Compute units that resident kernels of this process hold, per device.  Blocks of two such
 // kernels that cannot all run at once would wait for each other until their waits run out, so
@@ -1063,6 +1069,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     SgsResidentView rv{};
     ResidentTicket ticket;
     bool resident = !noResident() && sgs_resident_fits(n, P.wmax, ctx->n_cu, &rv.blocks);
+    const int quota = residentQuota();
     if (resident) {
         const size_t words = resident_sums(rv.blocks);
         W.pub.alloc(6 * (size_t)n);
@@ -1075,7 +1082,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     }
     for (;;) {
         const bool here = resident && ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
-        const long long todo = std::min<long long>(here ? RESIDENT_QUOTA : chunk, maxit - (k - base));
+        const long long todo = std::min<long long>(here ? quota : chunk, maxit - (k - base));
         if (todo <= 0) {
             out.done = 2;
             out.iters = k - base;
@@ -1268,7 +1275,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             rv.stale = w.slots.p + words;
             rv.blocks = plan.blocks;
             rv.rows = plan.rows;
-            rv.quota = RESIDENT_QUOTA;
+            rv.quota = residentQuota();
             rv.spin = residentSpin();
             rv.x64 = x;
         }

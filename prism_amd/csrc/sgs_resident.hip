@@ -134,9 +134,12 @@ __global__ void __launch_bounds__(BS) k_sgs_resident(SgsView V, SgsResidentView 
     SgsState* st = V.st;
     const int tid = threadIdx.x, lane = tid & 63, G = R.blocks, n = V.n, nc = V.nc;
     const int lb = (int)blockIdx.x < G ? (int)blockIdx.x : G;
-    if (st->done | st->flag | st->stuck) return;  // the same value in every thread of the grid
-    if (tid == 0) fail = 0;
+    // first of all, whatever else this launch does: the next one takes these words as unwritten
     if (tid < RES_LINE * (lb < G ? 1 : RES_COPIES)) post(&R.stale[RES_LINE * lb + tid], MARK);
+    // done and flag: the same values in every thread of the grid, as a launch writes them only after
+    // a round of totals.  stuck can be new here: then this launch's results count for nothing.
+    if (st->done | st->flag | st->stuck) return;
+    if (tid == 0) fail = 0;
     // totals of the last X (or the seed), as the first kernel of an iteration forms them
     double red[3];
 #pragma unroll
@@ -305,6 +308,13 @@ __global__ void __launch_bounds__(BS) k_sgs_resident(SgsView V, SgsResidentView 
         markSums(LINE_X, 2 * SUB);
         rho_old = rho;
         ++m;
+    }
+    // An event of the first test, before any exchange: one round, so that every block has read the
+    // event words and marked its stale ones before block 0 writes the event.
+    if (m == 0) {
+        const double none[2] = {0.0, 0.0};
+        double all[2];
+        if (!totals<2>(S, LINE_X, none, all, own)) return;
     }
     if (m > 0 && ok) {
         V.x[i] = x;

@@ -178,6 +178,58 @@ def test_sgs_same_bits_as_its_launches(hip, monkeypatch, n, row):
     assert np.linalg.norm(b - A @ x1) <= 2e-12 * np.linalg.norm(b)
 
 
+def broken_down(n, sgs):
+    """2 x 2 blocks on which rho is exactly zero after the first iteration (from b, which has no
+    second components, s and t have none of the first): A M^-1 has the blocks
+    [[1, 0], [k, h]] with (k, h) = (1/8, 3/4) and (-1/8, 5/4) in turn, so the first iteration
+    leaves a residual.  sgs: A has those blocks after preconditioning ([[1, a], [1/2, 1]], a = +-1/2)."""
+    odd = np.arange(n // 2) % 2 == 1
+    d, low, up = np.ones(n), np.zeros(n - 1), np.zeros(n - 1)
+    if sgs:
+        low[::2], up[::2] = 0.5, np.where(odd, -0.5, 0.5)
+    else:
+        d[1::2], low[::2] = np.where(odd, 1.25, 0.75), np.where(odd, -0.125, 0.125)
+    A = sp.diags([low, d, up], [-1, 0, 1], format="csr")
+    A.eliminate_zeros()
+    b = np.zeros(n)
+    b[::2] = 1.0
+    return A, b
+
+
+@pytest.mark.parametrize("quota", [1, 2, 128])
+@pytest.mark.parametrize("n", [4, 1026, 40000, 130560])
+@pytest.mark.parametrize("precond", [None, "sgs"])
+def test_breakdown_at_a_launch_boundary(hip, monkeypatch, precond, n, quota):
+    """The restart after a rho breakdown that a launch finds in its first test (quota 1: that
+    launch ends before its blocks have exchanged anything), and in a later one."""
+    print(f"case resident breakdown {precond} {n} {quota}", flush=True)
+    A, b = broken_down(n, precond == "sgs")
+    monkeypatch.setenv("PRISM_KRYLOV_QUOTA", str(quota))
+    xs, rs = [], []
+    for resident in "10":
+        monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", resident)
+        out = []
+        xs.append(P.solver.BiCGSTAB(tol=1e-12, precond=precond).step(matrix(hip, A), np.zeros(n), b, out))
+        rs.append(out[0])
+    np.testing.assert_array_equal(xs[0], xs[1])
+    assert [(r.krylov_iters, r.restarts, r.converged) for r in rs] == [(rs[0].krylov_iters, 1, 1)] * 2
+    assert np.linalg.norm(b - A @ xs[0]) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("quota", [1, 2, 3])
+@pytest.mark.parametrize("precision,precond", [("fp64", None), ("fp32", "jacobi"), ("fp64", "sgs")])
+@pytest.mark.parametrize("name", ["dia7_4095", "sell8_640", "sell5_513"])
+def test_state_handed_from_launch_to_launch(hip, monkeypatch, name, precision, precond, quota):
+    print(f"case resident hand-over {name} {precision} {precond} {quota}", flush=True)
+    A = SYSTEMS[name]
+    monkeypatch.setenv("PRISM_KRYLOV_QUOTA", str(quota))
+    x1, b, r1, used = solve(hip, A, monkeypatch, True, precision=precision, precond=precond)
+    x0, _, r0, _ = solve(hip, A, monkeypatch, False, precision=precision, precond=precond)
+    assert used
+    np.testing.assert_array_equal(x1, x0)
+    assert (r1.krylov_iters, r1.refinements, r1.restarts) == (r0.krylov_iters, r0.refinements, r0.restarts)
+
+
 def test_sgs_wait_that_runs_out_falls_back(hip, monkeypatch):
     print("case resident sgs spin", flush=True)
     monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
