@@ -422,6 +422,34 @@ void requireFaceValueBCs(const prism_field& f, const char* who) {
 // 128 x 128 cells (64 a level) 0.43 against 2.9 ms, 400 x 400 (200) 3.6 against 12.4, 24^3 x 6
 // tetrahedra (864) 1.24 against 1.10, 64^3 (1380) 6.2 against 4.1.
 constexpr int GG_SWEEP_WIDTH = 512;
+// Scratch of that sweep at most (it is kept with the mesh, 360 bytes a cell): a longer duct
+// takes the level launches, which need none.
+constexpr size_t GG_SWEEP_BYTES = size_t(1) << 30;
+
+// True when the mesh takes the sweep in one workgroup: its buffers are then there.  Where they
+// do not fit the device's memory it takes the level launches.
+bool prepareGGSweep(prism_mesh& m) {
+    const int64_t n = m.h.n;
+    const size_t faces = gg_sweep_faces();
+    int most = 0;
+    for (int64_t c = 0; c < n; ++c) most = std::max(most, m.h.cf_off[c + 1] - m.h.cf_off[c]);
+    if (most > gg_sweep_faces() || n > (int64_t)GG_SWEEP_WIDTH * ((int64_t)m.h.gg_off.size() - 1)) return false;
+    if (faces * n * (7 * sizeof(double) + sizeof(int32_t)) > GG_SWEEP_BYTES) return false;
+    try {
+        m.gg_lower.alloc(faces * n);
+        m.gg_terms.alloc(7 * faces * n);
+        m.gg_doff.upload(m.h.gg_off, m.ctx->stream);
+    } catch (const Error& e) {
+        if (e.code != PRISM_ERR_NOMEM) throw;
+        (void)hipGetLastError();  // or the next launch reports it
+        m.gg_lower.reset();
+        m.gg_terms.reset();
+        m.gg_doff.reset();
+        return false;
+    }
+    m.ctx->sync();
+    return true;
+}
 
 // Lazily refreshed gradient (gradient.h:26-31): recompute on first use after a write.
 void ensureGrad(prism_field& f) {
@@ -437,17 +465,7 @@ void ensureGrad(prism_field& f) {
     } else {
         const auto& off = m->h.gg_off;
         const int32_t levels = (int32_t)off.size() - 1;
-        if (m->gg_sweep < 0) {
-            int faces = 0;
-            for (int64_t c = 0; c < n; ++c) faces = std::max(faces, m->h.cf_off[c + 1] - m->h.cf_off[c]);
-            m->gg_sweep = faces <= gg_sweep_faces() && n <= (int64_t)GG_SWEEP_WIDTH * levels;
-            if (m->gg_sweep) {
-                m->gg_doff.upload(off, L.stream);
-                m->gg_lower.alloc((size_t)gg_sweep_faces() * n);
-                m->gg_terms.alloc(7 * (size_t)gg_sweep_faces() * n);
-                m->ctx->sync();
-            }
-        }
+        if (m->gg_sweep < 0) m->gg_sweep = prepareGGSweep(*m) ? 1 : 0;
         if (m->gg_sweep)
             launch_grad_gg_sweep(L, m->dm, s, m->gg_cells.p, m->gg_doff.p, levels, m->gg_lower.p, m->gg_terms.p, f.g.p,
                                  f.g.p + n, f.g.p + 2 * n);
