@@ -19,6 +19,7 @@
 #include <limits>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -779,7 +780,8 @@ struct prism_csr {
     int wmax{0};          // entries of the widest sliced-ELL slice
     bool all_diag{true};  // every row stores its diagonal entry
     DevBuf<double> val;
-    DevBuf<double> io[3];  // vectors of the calls on host arrays
+    DevBuf<double> io[3];  // vectors of the calls on host arrays, one call at a time
+    std::mutex io_use;
     Workspace ws;
     SgsCache sgs;
 };
@@ -2314,6 +2316,7 @@ API int prism_csr_create(prism_ctx* ctx, int64_t n, const int64_t* rp, const int
 API int prism_csr_destroy(prism_csr* a) { return guard([&] { delete a; }); }
 API int prism_csr_spmv(prism_csr* a, const double* x, double* y) {
     return guard([&] {
+        std::lock_guard<std::mutex> use(a->io_use);
         DevBuf<double>&dx = a->io[0], &dy = a->io[1];
         dx.upload(x, a->n, a->ctx->stream);
         dy.alloc(a->n);
@@ -2324,6 +2327,7 @@ API int prism_csr_spmv(prism_csr* a, const double* x, double* y) {
 }
 API int prism_csr_jacobi_step(prism_csr* a, const double* b, const double* xin, double* xout) {
     return guard([&] {  // jacobi.cpp:5-9: x + D^-1 (b - A x), on the device
+        std::lock_guard<std::mutex> use(a->io_use);
         DevBuf<double>&db = a->io[0], &dx = a->io[1], &dy = a->io[2];
         db.upload(b, a->n, a->ctx->stream);
         dx.upload(xin, a->n, a->ctx->stream);
@@ -2337,6 +2341,7 @@ API int prism_csr_bicgstab(prism_csr* a, const double* b, const double* xin, dou
                            const prism_solve_params* p, prism_solve_result* r) {
     return guard([&] {
         if (!a || !p || !b || !xin || !xout) fail(PRISM_ERR_INVALID, "BiCGSTAB::step: null argument");
+        std::lock_guard<std::mutex> use(a->io_use);
         DevBuf<double>&db = a->io[0], &dx = a->io[1];
         db.upload(b, a->n, a->ctx->stream);
         dx.upload(xin, a->n, a->ctx->stream);
