@@ -211,6 +211,8 @@ struct prism_mesh {
     DevBuf<double> pts;  // point values of the last export (grows to the widest field exported)
     int wmax{0};         // entries of the widest sliced-ELL slice
     // Green-Gauss sweep in one workgroup: -1 not looked at yet; its level offsets and scratch
+    // (the mesh's fields share them: gg_use is held until a sweep's launches are in the stream)
+    std::mutex gg_use;
     int gg_sweep{-1};
     DevBuf<int32_t> gg_doff, gg_lower;
     DevBuf<double> gg_terms;
@@ -466,6 +468,7 @@ void ensureGrad(prism_field& f) {
     } else {
         const auto& off = m->h.gg_off;
         const int32_t levels = (int32_t)off.size() - 1;
+        std::lock_guard<std::mutex> use(m->gg_use);
         if (m->gg_sweep < 0) m->gg_sweep = prepareGGSweep(*m) ? 1 : 0;
         if (m->gg_sweep)
             launch_grad_gg_sweep(L, m->dm, s, m->gg_cells.p, m->gg_doff.p, levels, m->gg_lower.p, m->gg_terms.p, f.g.p,

@@ -50,3 +50,29 @@ def test_products_of_one_matrix(hip, n):
             assert np.abs(P.solver.Jacobi().step(A, xs[2], xs[1]) - exact).max() <= bound
 
     together(lambda: products(xs[0]), lambda: products(xs[1]), steps)
+
+
+def test_green_gauss_fields_of_one_mesh(hip):
+    """The sweep in one workgroup shares its scratch among the mesh's fields."""
+    print("case threads gradients", flush=True)
+    data = P.box(60, 50, 1, jitter=0.0)
+    bcs = {s: {"T": ("fixed", 0.5), "f": ("fixed", 0.25)} for s in data.patch_names}
+    rng = np.random.default_rng(8)
+    values = {name: rng.standard_normal((20, data.n_cells)) for name in ("T", "f")}
+
+    def sweeps(m, name, out):
+        field = m.scalar(name, values=values[name][0])
+        for v in values[name]:
+            field.values = v
+            out.append(field.grad())
+
+    def mesh():
+        return P.Mesh(hip, data, bcs, [("T", "scalar", "greenGauss"), ("f", "scalar", "greenGauss")])
+
+    alone, shared = {"T": [], "f": []}, {"T": [], "f": []}
+    one, two = mesh(), mesh()
+    for name in alone:
+        sweeps(one, name, alone[name])
+    together(*[lambda name=name: sweeps(two, name, shared[name]) for name in shared])
+    for name in alone:
+        np.testing.assert_array_equal(shared[name], alone[name])
