@@ -126,6 +126,7 @@ struct prism_ctx {
     std::map<std::string, std::pair<int64_t, double>> stats;
     std::vector<std::string> order;
     void* hks{nullptr};  // pinned: the scalars last read back (KrylovScalars or SgsState)
+    std::mutex hks_use;
     unsigned char* scratch{nullptr};  // this device's static scratch array (scratch_address)
     int n_cu{0};                      // compute units of the device
 
@@ -177,6 +178,14 @@ struct prism_ctx {
         pending.clear();
     }
     void sync() { HIPCHECK(hipStreamSynchronize(stream)); }
+    // A scalar block of the device, once the stream has reached this point.
+    template <typename S>
+    S readBack(const S* src) {
+        std::lock_guard<std::mutex> use(hks_use);
+        launch_read_back(launch(), src, hks, sizeof(S));
+        sync();
+        return *static_cast<S*>(hks);
+    }
 };
 
 // --------------------------------------------------- SGS preconditioner plan ----
@@ -996,11 +1005,7 @@ hipGraphExec_t iterationPair(Workspace& w, const Launch& L, KView<T>& kv, SetIte
     return g.exec;
 }
 
-KrylovScalars pollScalars(prism_ctx* ctx, Workspace& w) {
-    launch_read_back(ctx->launch(), w.ks.p, ctx->hks, sizeof(KrylovScalars));
-    HIPCHECK(hipStreamSynchronize(ctx->stream));
-    return *static_cast<KrylovScalars*>(ctx->hks);
-}
+KrylovScalars pollScalars(prism_ctx* ctx, Workspace& w) { return ctx->readBack(w.ks.p); }
 
 // One BiCGSTAB step x <- BiCGSTAB(A, b, x) (bicgstab.cpp:7-9 semantics: a full solve from the
 // current guess).  precision 0: FP64.  precision 1: FP32 iteration with FP64 reliable updates
@@ -1078,11 +1083,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     V.part_v = W.part_v.p;
     V.part_t = W.part_t.p;
     V.st = W.st.p;
-    auto poll = [&] {
-        launch_read_back(L, W.st.p, ctx->hks, sizeof(SgsState));
-        ctx->sync();
-        return *static_cast<SgsState*>(ctx->hks);
-    };
+    auto poll = [&] { return ctx->readBack(W.st.p); };
     if (poll().bad_diag) fail(PRISM_ERR_RUNTIME, "SGS preconditioner: a diagonal entry is zero or not finite");
     launch_sgs_seed(L, V, true);
     const long long maxit = p.max_iters > 0 ? p.max_iters : 2 * (long long)n;

@@ -76,3 +76,33 @@ def test_green_gauss_fields_of_one_mesh(hip):
     together(*[lambda name=name: sweeps(two, name, shared[name]) for name in shared])
     for name in alone:
         np.testing.assert_array_equal(shared[name], alone[name])
+
+
+@pytest.mark.parametrize("precond", [None, "sgs"])
+def test_solves_on_one_context(hip, precond):
+    """Each solve polls its own scalars, through the context's one pinned buffer."""
+    print(f"case threads solves {precond}", flush=True)
+    systems, alone = [], []
+    for n in (900, 5000):
+        rng = np.random.default_rng(n)
+        A = sp.diags([rng.uniform(-1.0, 0.3, n - o) for o in (1, 22)] * 2, (1, 22, -1, -22), format="csr")
+        A = (A + sp.diags(1.02 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.01)).tocsr()
+        A.sort_indices()
+        b = rng.standard_normal(n)
+
+        def solves(times, M=P.Matrix(hip, A.indptr, A.indices, A.data), b=b):
+            s = P.solver.BiCGSTAB(tol=1e-12, precond=precond)
+            return [s.step(M, np.zeros(len(b)), b) for _ in range(times)]
+
+        systems.append(solves)
+        alone.append(solves(1)[0])
+        assert np.linalg.norm(b - A @ alone[-1]) <= 2e-12 * np.linalg.norm(b)
+    got = [None, None]
+
+    def run(k):
+        got[k] = systems[k](10)
+
+    together(lambda: run(0), lambda: run(1))
+    for xs, x in zip(got, alone):
+        for y in xs:
+            np.testing.assert_array_equal(y, x)
