@@ -9,7 +9,6 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 #include <chrono>
 #include <cmath>
@@ -29,6 +28,7 @@
 #include "krylov.h"
 #include "output.h"
 #include "resident.h"
+#include "resident_ticket.h"
 #include "sgs.h"
 
 using namespace prism_hip;
@@ -939,40 +939,6 @@ int residentQuota() {
     const int q = e ? std::atoi(e) : 0;
     return q > 0 ? std::min(q, RESIDENT_QUOTA) : RESIDENT_QUOTA;
 }
-
-// Compute units that resident kernels of this process hold, per device.  Blocks of two such
-// kernels that cannot all run at once would wait for each other until their waits run out, so
-// a launch that does not fit beside those in flight is not made (the caller takes the
-// three-kernel iteration for that chunk).
-class ResidentTicket {
-    static std::atomic<int>& held(int device) {
-        static std::atomic<int> h[64];
-        return h[device & 63];
-    }
-    std::atomic<int>* at_{nullptr};
-    int blocks_{0};
-
-public:
-    bool take(int device, int blocks, int n_cu) {
-        give();
-        std::atomic<int>& h = held(device);
-        if (h.fetch_add(blocks) + blocks > n_cu) {
-            h.fetch_sub(blocks);
-            return false;
-        }
-        at_ = &h;
-        blocks_ = blocks;
-        return true;
-    }
-    void give() {
-        if (at_) at_->fetch_sub(blocks_);
-        at_ = nullptr;
-    }
-    ResidentTicket() = default;
-    ResidentTicket(const ResidentTicket&) = delete;
-    ResidentTicket& operator=(const ResidentTicket&) = delete;
-    ~ResidentTicket() { give(); }
-};
 
 bool graphsEnabled() {
     static const bool on = [] {
