@@ -1071,14 +1071,14 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
         rv.spin = residentSpin();
     }
     for (;;) {
-        const bool here = resident && ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
-        const long long todo = std::min<long long>(here ? quota : chunk, maxit - (k - base));
+        const long long todo = std::min<long long>(resident ? quota : chunk, maxit - (k - base));
         if (todo <= 0) {
             out.done = 2;
             out.iters = k - base;
             break;
         }
-        if (here) {
+        if (resident) {
+            ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
             rv.quota = (int)todo;
             launch_sgs_resident(L, V, rv, P.wmax, k, fresh);
             std::swap(rv.line, rv.stale);
@@ -1435,7 +1435,8 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             }
             last_iter = s.nit;
             last_rr = s.rr;
-            if (plan.blocks > 0 && ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu)) {
+            if (plan.blocks > 0) {
+                ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu);
                 launch_resident<T>(L, kv, rv, plan);
                 resident_last = true;
                 std::swap(rv.slots, rv.stale);

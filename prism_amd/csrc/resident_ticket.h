@@ -3,13 +3,17 @@
 // A resident kernel ends only if all of its blocks run at the same time, and almost every
 // instance needs a compute unit for each (its registers leave no room for a second block).  Blocks
 // of two such kernels that cannot all run would wait for each other until their waits run out,
-// so a launch that does not fit beside those in flight is not made.
+// so a launch waits for its turn, in the order of asking: until it fits beside those in flight, a
+// launch of 128 iterations (1 to 4 ms) or two.  (The launches of the single kernels could go
+// on at once, but they sum in another order from 130,561 rows on: which of the two a
+// solve got would then depend on what other threads did at that moment, and so would its bits.)
 //
 // Blocks go to the XCDs in turn, so b blocks take up to ceil(b / 8) compute units of each: that is
 // what is counted.  (Counted in blocks, 132 and 124 of them would fit 256 units; four XCDs would
 // get 17 + 16 for their 32.)
 #pragma once
 
+#include <condition_variable>
 #include <mutex>
 
 namespace prism_hip {
@@ -19,7 +23,9 @@ constexpr int XCDS = 8;
 class ResidentTicket {
     struct Device {
         std::mutex use;
+        std::condition_variable turn;
         int held{0};  // compute units of an XCD
+        unsigned long long asked{0}, served{0};
     };
     static Device& device(int i) {
         static Device d[64];
@@ -29,23 +35,29 @@ class ResidentTicket {
     int share_{0};
 
 public:
-    // True when a kernel of `blocks` blocks fits beside those in flight on the device (one that
-    // is alone always does: its plan has no more blocks than compute units).
-    bool take(int dev, int blocks, int n_cu) {
+    // Compute units of an XCD that `blocks` blocks take, and whether that many fit beside `held`
+    // (a kernel alone always does: its plan has no more blocks than compute units).
+    static int share(int blocks) { return (blocks + XCDS - 1) / XCDS; }
+    static bool fits(int held, int share, int n_cu) { return held == 0 || held + share <= n_cu / XCDS; }
+
+    void take(int dev, int blocks, int n_cu) {
         give();
-        const int share = (blocks + XCDS - 1) / XCDS;
+        const int want = share(blocks);
         Device& d = device(dev);
-        std::lock_guard<std::mutex> lock(d.use);
-        if (d.held > 0 && d.held + share > n_cu / XCDS) return false;
-        d.held += share;
+        std::unique_lock<std::mutex> lock(d.use);
+        const unsigned long long mine = d.asked++;
+        d.turn.wait(lock, [&] { return mine == d.served && fits(d.held, want, n_cu); });
+        ++d.served;
+        d.held += want;
         at_ = &d;
-        share_ = share;
-        return true;
+        share_ = want;
+        d.turn.notify_all();
     }
     void give() {
         if (!at_) return;
         std::lock_guard<std::mutex> lock(at_->use);
         at_->held -= share_;
+        at_->turn.notify_all();
         at_ = nullptr;
     }
     ResidentTicket() = default;

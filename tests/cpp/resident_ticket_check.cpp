@@ -1,7 +1,12 @@
 // Which resident kernels may be in flight together (prism_amd/csrc/resident_ticket.h): the blocks of
-// every set that is let in, dealt to the XCDs in turn from any one on, fit their compute units.
+// every set that is let in, dealt to the XCDs in turn from any one on, fit their compute
+// units; the others wait, and are served in the order of asking.
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <thread>
+#include <vector>
 
 #include "../../prism_amd/csrc/resident_ticket.h"
 
@@ -14,28 +19,73 @@ static void check(bool ok, const char* what, int a, int b) {
     std::exit(1);
 }
 
+static void settle() { std::this_thread::sleep_for(std::chrono::milliseconds(50)); }
+
 int main() {
     const int cu = 256;
     for (int a = 1; a <= cu; ++a)
         for (int b = 1; b <= cu; ++b) {
-            ResidentTicket s, t;
-            check(s.take(0, a, cu), "a kernel alone is refused", a, 0);
-            const bool both = t.take(0, b, cu);
+            const bool both = ResidentTicket::fits(ResidentTicket::share(a), ResidentTicket::share(b), cu);
             // most blocks that an XCD of 32 units can get
             const int worst = (a + XCDS - 1) / XCDS + (b + XCDS - 1) / XCDS;
             check(!both || worst <= cu / XCDS, "more blocks than an XCD has units", a, b);
             check(both || worst > cu / XCDS, "refused though it fits", a, b);
-            ResidentTicket other;
-            check(other.take(1, cu, cu), "another device's kernels are counted", a, b);
+            check(ResidentTicket::fits(0, ResidentTicket::share(a), b), "a kernel alone is refused", a, b);
         }
     {
-        ResidentTicket s, t;
-        check(s.take(0, 132, cu) && !t.take(0, 124, cu), "17 + 16 of 32 units", 132, 124);
-        s.give();
-        check(t.take(0, 124, cu), "units given back are not free", 132, 124);
-        check(t.take(0, cu, cu), "a ticket taken again keeps its first units", cu, 0);
+        // 132 and 124 blocks want 17 + 16 of 32 units: the second waits, and what asks after it
+        // (small enough to go at once) does not pass it
+        ResidentTicket first;
+        first.take(0, 132, cu);
+        std::atomic<int> order{0};
+        int big = 0, small = 0, elsewhere = 0;
+        std::thread t([&] {
+            ResidentTicket s;
+            s.take(0, 124, cu);
+            big = ++order;
+            settle();
+        });
+        settle();
+        std::thread u([&] {
+            ResidentTicket s;
+            s.take(0, 8, cu);
+            small = ++order;
+        });
+        settle();
+        check(order == 0, "let in beside 132 blocks", 132, 124);
+        std::thread v([&] {
+            ResidentTicket s;
+            s.take(1, cu, cu);
+            elsewhere = 1;
+        });
+        v.join();
+        check(elsewhere == 1, "another device's kernels are counted", 1, 0);
+        first.give();
+        t.join();
+        u.join();
+        check(big == 1 && small == 2, "order of asking", big, small);
+        first.take(0, cu, cu);
+        first.take(0, cu, cu);  // taken again: its first units are given back
     }
-    ResidentTicket t;
-    check(t.take(0, 7, 6), "a device of few units, alone", 7, 6);
+    {
+        // never more than the units of an XCD at once
+        std::atomic<int> held{0}, worst{0}, rounds{0};
+        std::vector<std::thread> ts;
+        for (int k = 0; k < 6; ++k)
+            ts.emplace_back([&, k] {
+                ResidentTicket s;
+                for (int i = 0; i < 500; ++i) {
+                    const int blocks = 1 + (37 * i + 91 * k) % cu, units = ResidentTicket::share(blocks);
+                    s.take(2, blocks, cu);
+                    const int h = held += units;
+                    if (h > worst) worst = h;
+                    held -= units;
+                    s.give();
+                    ++rounds;
+                }
+            });
+        for (auto& t : ts) t.join();
+        check(rounds == 3000 && worst <= cu / XCDS, "units held at once", rounds, worst);
+    }
     std::puts("ok");
 }

@@ -140,8 +140,8 @@ def test_wait_that_runs_out_falls_back(hip, monkeypatch, precision):
 
 
 def test_two_threads_share_the_device(hip, monkeypatch):
-    """Two contexts solve at once; together their blocks exceed the device, so one of them takes
-    the three-kernel iteration now and then: the same bits either way."""
+    """Two contexts solve at once; together their blocks exceed the device, so their launches take
+    turns: the bits of a solve alone."""
     print("case resident two threads", flush=True)
     monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
     A = diagonals(100000, (-2000, -50, -1, 1, 50, 2000))
@@ -161,6 +161,35 @@ def test_two_threads_share_the_device(hip, monkeypatch):
         t.join()
     for k in range(2):
         for x in out[k]:
+            np.testing.assert_array_equal(x, alone)
+
+
+@pytest.mark.parametrize("n,offsets,precision,precond", [
+    (50000, (-2000, -50, -1, 1, 50, 2000), "fp64", None),      # 98 blocks each: both run
+    (150000, (-2000, -50, -1, 1, 50, 2000), "fp64", None),     # two rows per thread
+    (64 * 64 * 40, (-4096, -64, -1, 1, 64, 4096), "fp32", None),  # the single kernels are the packed ones
+    (100000, (-50, -1, 1, 50), "fp64", "sgs")])
+def test_threads_do_not_change_the_bits(hip, monkeypatch, n, offsets, precision, precond):
+    print(f"case resident threads {n} {precision} {precond}", flush=True)
+    monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
+    A = diagonals(n, offsets)
+    b = np.random.default_rng(2).standard_normal(n)
+    s = P.solver.BiCGSTAB(tol=1e-12, precision=precision, precond=precond)
+    alone = s.step(matrix(hip, A), np.zeros(n), b)
+    out = [[] for _ in range(3)]
+
+    def work(xs):
+        M = matrix(P.Backend.hip(0), A)
+        xs.extend(s.step(M, np.zeros(n), b) for _ in range(4))
+
+    ts = [threading.Thread(target=work, args=(xs,)) for xs in out]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for xs in out:
+        assert len(xs) == 4
+        for x in xs:
             np.testing.assert_array_equal(x, alone)
 
 
