@@ -129,6 +129,7 @@ struct prism_ctx {
     std::mutex hks_use;
     unsigned char* scratch{nullptr};  // this device's static scratch array (scratch_address)
     int n_cu{0};                      // compute units of the device
+    ResidentRest rest;                // of the resident kernels, after a wait that ran out
 
     Launch launch() {
         Launch L;
@@ -932,6 +933,10 @@ unsigned residentSpin() {
     return e && std::atol(e) > 0 ? (unsigned)std::atol(e) : 1u << 20;
 }
 
+double seconds() {
+    return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
 // Iterations of one resident launch at most (PRISM_KRYLOV_QUOTA: fewer, read per solve).
 constexpr int RESIDENT_QUOTA = 128;
 int residentQuota() {
@@ -1058,7 +1063,8 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     int fresh = 1, chunk = 4;
     SgsResidentView rv{};
     ResidentTicket ticket;
-    bool resident = !noResident() && sgs_resident_fits(n, P.wmax, ctx->n_cu, &rv.blocks);
+    double launched = 0.0;  // when the last resident launch was made
+    bool resident = !noResident() && sgs_resident_fits(n, P.wmax, ctx->n_cu, &rv.blocks) && ctx->rest.over(seconds());
     const int quota = residentQuota();
     if (resident) {
         const size_t words = resident_sums(rv.blocks);
@@ -1081,6 +1087,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
             ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
             rv.quota = (int)todo;
             launch_sgs_resident(L, V, rv, P.wmax, k, fresh);
+            launched = seconds();
             std::swap(rv.line, rv.stale);
         } else {
             for (long long j = 0; j < todo; ++j) launch_sgs_iteration(L, V, k + j, j == 0 ? fresh : 0);
@@ -1089,6 +1096,8 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
         const SgsState s = poll();
         ticket.give();
         if (s.stuck) {  // a wait of the resident kernel ran out: on from this x without it
+            const double now = seconds();
+            ctx->rest.ranOut(now - launched, now);
             resident = false;
             h.s[0] = h.s[1];  // the start state at either parity
             HIPCHECK(hipMemcpyAsync(W.st.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
@@ -1096,6 +1105,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
             fresh = 1;
             continue;
         }
+        if (resident) ctx->rest.endedWell();
         if (s.done) {
             out.done = s.done;
             out.iters = s.k_event - base;
@@ -1250,7 +1260,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         ResidentPlan plan;
         ResidentView<T> rv{};
         ResidentTicket ticket;
-        if (three && !w.scratch && (sizeof(T) == 8 || kv.diff) && !noResident())
+        if (three && !w.scratch && (sizeof(T) == 8 || kv.diff) && !noResident() && ctx->rest.over(seconds()))
             plan = resident_plan<T>(A.n, dia, dia ? A.ndia : A.wmax, ctx->n_cu);
         if (plan.blocks > 0) {
             DevBuf<T>* pub;
@@ -1335,14 +1345,18 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         double last_true = INFINITY;
         bool forced = false;  // the pending reliable update was forced by stagnation
         bool resident_last = false;  // the launch before this poll was the resident kernel
+        double launched = 0.0;       // when it was made (its code is loaded by then)
         int stalls = 0;       // forced updates in a row that did not lower the FP64 residual
         for (;;) {
             KrylovScalars s = pollScalars(ctx, w);
             ticket.give();
             const bool flushed = resident_last && s.flag;  // by the resident kernel
+            if (resident_last && !s.stuck) ctx->rest.endedWell();
             resident_last = false;
             if (s.stuck) {  // a wait of the resident kernel ran out: on from this x without it
                 if (traceEnabled()) std::fprintf(stderr, "krylov n=%d: resident kernel stuck\n", A.n);
+                const double now = seconds();
+                ctx->rest.ranOut(now - launched, now);
                 plan.blocks = 0;
                 if constexpr (sizeof(T) == 4) launch_flush(L, A.n, x, kv.x);
                 launch_reset_events(L, w.ks.p, true, false);
@@ -1438,6 +1452,7 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             if (plan.blocks > 0) {
                 ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu);
                 launch_resident<T>(L, kv, rv, plan);
+                launched = seconds();
                 resident_last = true;
                 std::swap(rv.slots, rv.stale);
             } else if (three) {

@@ -13,6 +13,7 @@
 // get 17 + 16 for their 32.)
 #pragma once
 
+#include <algorithm>
 #include <condition_variable>
 #include <mutex>
 
@@ -64,6 +65,33 @@ public:
     ResidentTicket(const ResidentTicket&) = delete;
     ResidentTicket& operator=(const ResidentTicket&) = delete;
     ~ResidentTicket() { give(); }
+};
+
+// When a context takes resident kernels again after a wait that ran out: their blocks do not
+// run together then, because another process (whose kernels the ticket does not see) holds compute
+// units, and the next solves would lose the same time, up to 2^20 polls (several tenths
+// of a second) for a solve of milliseconds.  They stay off for 8 times the time lost, twice as long
+// each further time in a row: at most a ninth of the time goes into such waits.  Times in
+// seconds, of one steady clock.
+class ResidentRest {
+    std::mutex use_;
+    double until_{0.0}, factor_{FIRST};
+
+public:
+    static constexpr double FIRST = 8.0, MOST = 1024.0;
+    bool over(double now) {
+        std::lock_guard<std::mutex> lock(use_);
+        return now >= until_;
+    }
+    void ranOut(double lost, double now) {
+        std::lock_guard<std::mutex> lock(use_);
+        until_ = now + factor_ * lost;
+        factor_ = std::min(2.0 * factor_, MOST);
+    }
+    void endedWell() {
+        std::lock_guard<std::mutex> lock(use_);
+        factor_ = FIRST;
+    }
 };
 
 }  // namespace prism_hip

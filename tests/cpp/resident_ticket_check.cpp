@@ -87,5 +87,27 @@ int main() {
         for (auto& t : ts) t.join();
         check(rounds == 3000 && worst <= cu / XCDS, "units held at once", rounds, worst);
     }
+    {
+        // waits that run out after 0.4 s each, in a process that solves without a pause
+        prism_hip::ResidentRest rest;
+        check(rest.over(0.0), "off at the start", 0, 0);
+        double now = 100.0, lost = 0.0;
+        int waits = 0;
+        while (now < 1100.0) {
+            if (rest.over(now)) {
+                now += 0.4;
+                lost += 0.4;
+                ++waits;
+                rest.ranOut(0.4, now);
+                check(!rest.over(now) && !rest.over(now + 3.1), "on again at once", waits, 0);
+            }
+            now += 0.005;  // a solve
+            check(lost <= 0.4 + (now - 100.0) / 9.0, "time lost", waits, (int)now);
+        }
+        check(waits >= 5 && waits <= 10, "waits in 1000 s", waits, 0);
+        rest.endedWell();
+        rest.ranOut(0.4, 5000.0);
+        check(!rest.over(5003.1) && rest.over(5003.3), "the first rest again", 0, 0);
+    }
     std::puts("ok");
 }

@@ -2,6 +2,7 @@
 exact solutions: with one row per thread both form every sum in the same order, so the
 solutions are the same bits; with more, each solution satisfies the system."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -137,6 +138,36 @@ def test_wait_that_runs_out_falls_back(hip, monkeypatch, precision):
     x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision)
     assert used and r.krylov_rel_residual <= 1e-12
     assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("precond,kernel", [(None, "bicgstab_resident_f64"), ("sgs", "sgs_resident")])
+def test_waits_that_run_out_are_remembered(hip, monkeypatch, precond, kernel):
+    """A context whose resident kernels gave up keeps off them for a multiple of the time lost,
+    longer each time, and takes them again afterwards."""
+    print(f"case resident rest {precond}", flush=True)
+    monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
+    monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
+    be = P.Backend.hip(0)
+    A = diagonals(5000, (-22, -1, 1, 22))
+    M, b = matrix(be, A), np.random.default_rng(9).standard_normal(5000)
+    s = P.solver.BiCGSTAB(tol=1e-12, precond=precond)
+
+    def launches(times):
+        be.set_timing(True)
+        be.reset_timing()
+        for _ in range(times):
+            x = s.step(M, np.zeros(5000), b)
+            assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+        n = be.kernel_stats().get(kernel, (0,))[0]
+        be.set_timing(False)
+        return n
+
+    # a context that forgets would launch one in each solve
+    assert 1 <= launches(200) < 200
+    monkeypatch.delenv("PRISM_KRYLOV_SPIN")
+    time.sleep(2.0)
+    assert launches(5) >= 5
+    be.close()
 
 
 def test_two_threads_share_the_device(hip, monkeypatch):
