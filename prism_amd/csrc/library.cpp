@@ -64,6 +64,20 @@ int guard(F&& f) {
 }
 [[noreturn]] void fail(int code, const std::string& m) { throw Error(code, m); }
 
+// Runs `allocate` for a path that another one can stand in for: false when the device has no
+// memory left for it.
+template <class F>
+bool roomFor(F&& allocate) {
+    try {
+        allocate();
+        return true;
+    } catch (const Error& e) {
+        if (e.code != PRISM_ERR_NOMEM) throw;
+        (void)hipGetLastError();  // or the next launch reports it
+        return false;
+    }
+}
+
 template <typename T>
 struct DevBuf {
     T* p{nullptr};
@@ -448,13 +462,12 @@ bool prepareGGSweep(prism_mesh& m) {
     for (int64_t c = 0; c < n; ++c) most = std::max(most, m.h.cf_off[c + 1] - m.h.cf_off[c]);
     if (most > gg_sweep_faces() || n > (int64_t)GG_SWEEP_WIDTH * ((int64_t)m.h.gg_off.size() - 1)) return false;
     if (faces * n * (7 * sizeof(double) + sizeof(int32_t)) > GG_SWEEP_BYTES) return false;
-    try {
+    const bool room = roomFor([&] {
         m.gg_lower.alloc(faces * n);
         m.gg_terms.alloc(7 * faces * n);
         m.gg_doff.upload(m.h.gg_off, m.ctx->stream);
-    } catch (const Error& e) {
-        if (e.code != PRISM_ERR_NOMEM) throw;
-        (void)hipGetLastError();  // or the next launch reports it
+    });
+    if (!room) {
         m.gg_lower.reset();
         m.gg_terms.reset();
         m.gg_doff.reset();
@@ -1066,10 +1079,12 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
     double launched = 0.0;  // when the last resident launch was made
     bool resident = !noResident() && sgs_resident_fits(n, P.wmax, ctx->n_cu, &rv.blocks) && ctx->rest.over(seconds());
     const int quota = residentQuota();
+    const size_t words = resident ? resident_sums(rv.blocks) : 0;
+    resident = resident && roomFor([&] {
+                   W.pub.alloc(6 * (size_t)n);
+                   W.lines.alloc(2 * words);
+               });
     if (resident) {
-        const size_t words = resident_sums(rv.blocks);
-        W.pub.alloc(6 * (size_t)n);
-        W.lines.alloc(2 * words);
         launch_resident_mark<double>(L, W.pub.p, W.pub.n, W.lines.p, W.lines.n);
         rv.pub = W.pub.p;
         rv.line = W.lines.p;
@@ -1262,13 +1277,16 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
         ResidentTicket ticket;
         if (three && !w.scratch && (sizeof(T) == 8 || kv.diff) && !noResident() && ctx->rest.over(seconds()))
             plan = resident_plan<T>(A.n, dia, dia ? A.ndia : A.wmax, ctx->n_cu);
+        DevBuf<T>* pub;
+        if constexpr (sizeof(T) == 8) pub = &w.d_pub;
+        else pub = &w.f_pub;
+        const size_t words = resident_sums(plan.blocks);
+        if (plan.blocks > 0 && !roomFor([&] {
+                pub->alloc(5 * (size_t)A.n);
+                w.slots.alloc(2 * words);
+            }))
+            plan.blocks = 0;
         if (plan.blocks > 0) {
-            DevBuf<T>* pub;
-            if constexpr (sizeof(T) == 8) pub = &w.d_pub;
-            else pub = &w.f_pub;
-            const size_t words = resident_sums(plan.blocks);
-            pub->alloc(5 * (size_t)A.n);
-            w.slots.alloc(2 * words);
             launch_resident_mark<T>(L, pub->p, pub->n, w.slots.p, w.slots.n);
             rv.pub = pub->p;
             rv.slots = w.slots.p;

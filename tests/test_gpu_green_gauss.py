@@ -1,12 +1,11 @@
 """The Green-Gauss sweep in one workgroup (narrow levels, among them levels wider than the
 workgroup) and as a launch for each level (wide ones), against the oracle's sequential sweep,
 twice: the second sweep starts from the first one's gradients."""
-import ctypes as C
-
 import numpy as np
 import pytest
 
 import prism_amd as P
+from devmem import full_device
 
 pytestmark = pytest.mark.gpu
 
@@ -44,25 +43,9 @@ def test_sweep_without_room_for_its_scratch(hip):
     meshes = [P.Mesh(hip, data, bcs, [("T", "scalar", "greenGauss")]) for _ in range(2)]
     fields = [m.scalar("T", values=values[0]) for m in meshes]
     expected = fields[0].grad()
-    rt = P.hip_lib().dll  # the HIP runtime's calls are found through the library that links it
-    held = []
-
-    def free():
-        f, t = C.c_size_t(), C.c_size_t()
-        assert rt.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
-        return f.value
-
-    try:
-        for chunk in (8 << 30, 512 << 20, 32 << 20):  # each as long as 96 MB remain
-            while free() >= chunk + (96 << 20):
-                p = C.c_void_p()
-                assert rt.hipMalloc(C.byref(p), C.c_size_t(chunk)) == 0
-                held.append(p)
-        assert free() < 360 * data.n_cells
+    with full_device(96 << 20) as left:
+        assert left < 360 * data.n_cells
         got = fields[1].grad()
-    finally:
-        for p in held:
-            rt.hipFree(p)
     assert np.abs(got - expected).max() <= 1e-13 * np.abs(expected).max()
     for f in fields:
         f.values = values[1]

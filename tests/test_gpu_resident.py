@@ -9,6 +9,7 @@ import pytest
 import scipy.sparse as sp
 
 import prism_amd as P
+from devmem import full_device
 
 pytestmark = pytest.mark.gpu
 
@@ -168,6 +169,28 @@ def test_waits_that_run_out_are_remembered(hip, monkeypatch, precond, kernel):
     time.sleep(2.0)
     assert launches(5) >= 5
     be.close()
+
+
+def test_without_room_for_the_exchange(hip, monkeypatch):
+    """A solve whose other buffers are there, on a device with at most 24 of the 24.9 MiB left that
+    the exchanged words take: the single kernels."""
+    print("case resident without room", flush=True)
+    n = 255 * 2560
+    A = diagonals(n, (-4096, -1, 1, 4096))
+    M, b = matrix(hip, A), np.random.default_rng(9).standard_normal(n)
+    s = P.solver.BiCGSTAB(tol=1e-12)
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "0")
+    expected = s.step(M, np.zeros(n), b)
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "1")
+    with full_device(8 << 20) as left:
+        assert left < 5 * 8 * n
+        x = s.step(M, np.zeros(n), b)
+    np.testing.assert_array_equal(x, expected)  # the resident sums run in another order here
+    hip.set_timing(True)
+    hip.reset_timing()
+    s.step(M, np.zeros(n), b)
+    assert "bicgstab_resident_f64" in hip.kernel_stats()
+    hip.set_timing(False)
 
 
 def test_two_threads_share_the_device(hip, monkeypatch):
