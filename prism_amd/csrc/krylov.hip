@@ -271,6 +271,9 @@ __device__ inline T sellRow(const int* __restrict__ soff, const int* __restrict_
     const int o = soff[s];
     const int w = (soff[s + 1] - o) >> 6;  // >= 1: every row holds its diagonal
     switch (w) {
+    case 1: return sellExact<1, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
+    case 2: return sellExact<2, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
+    case 3: return sellExact<3, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
     case 4: return sellExact<4, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
     case 5: return sellExact<5, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
     case 6: return sellExact<6, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
@@ -278,23 +281,27 @@ __device__ inline T sellRow(const int* __restrict__ soff, const int* __restrict_
     case 8: return sellExact<8, T, REL, DIFF>(scol, srel, sbase, sval, o, lane, row, op);
     default: break;
     }
-    // other widths: eight slots at a time (past the last one, it again), their loads together
+    // wider: four slots at a time (past the last one, it again), their loads together.  V and T at
+    // 1.5 million rows, FP64, one slot / eight / four at a time: width 10 72 / 78 / 72 us, width 12
+    // 93 / 91 / 82 us, width 17 158 / 150 / 140 us; FP32, width 10 51 / 52 / 48 us, width 13
+    // 61 / 53 / 57 us.  Widths 1 to 3 in eights of these loads took 29 us where their own bodies take
+    // 25 us (width 2, FP64).
     T sum = T(0);
     const T xi = DIFF ? op(row) : T(0);
-    for (int k0 = 0; k0 < w; k0 += 8) {
-        int cj[8];
-        T vv[8], xv[8];
+    for (int k0 = 0; k0 < w; k0 += 4) {
+        int cj[4];
+        T vv[4], xv[4];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 4; ++q) {
             const int k = min(k0 + q, w - 1), p = (int)sellPos(o, w, k, lane);
             vv[q] = sval[p];
             if constexpr (REL) cj[q] = row + sbase[(o >> 6) + k] + (int)srel[p];
             else cj[q] = scol[p];
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) xv[q] = op(cj[q]);
+        for (int q = 0; q < 4; ++q) xv[q] = op(cj[q]);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 4; ++q) {
             if (k0 + q >= w) break;
             if (DIFF && cj[q] != row) sum += vv[q] * (xv[q] - xi);
             else if (DIFF != 2) sum += vv[q] * xv[q];

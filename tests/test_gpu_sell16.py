@@ -7,6 +7,7 @@ import os
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import prism_amd as P
 from prism_amd import cases
@@ -72,3 +73,29 @@ def test_16_bit_offsets_against_oracle(hip, ref, mesh_data):
     P.solver.BiCGSTAB(tol=1e-13).solve(cr["eqn"], 2, 1e-20)
     d = ch["T"].values - cr["T"].values
     assert np.linalg.norm(d) / np.linalg.norm(cr["T"].values) <= 1e-10
+
+
+@pytest.mark.parametrize("precision,bound", [("fp64", 1e-12), ("fp32", 1e-10)])
+@pytest.mark.parametrize("width", [1, 2, 3, 4, 8, 9, 10, 11, 12, 13, 17])
+def test_slice_widths(hip, monkeypatch, width, precision, bound):
+    """The single kernels' row products at every shape of their bodies: slices of one width, and of
+    smaller ones (every fifth row has half the entries), columns near (16 bits) and scattered."""
+    print(f"case slice width {width} {precision}", flush=True)
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "0")
+    n = 1000
+    for reach in (40, n):
+        rng = np.random.default_rng(width)
+        A = sp.lil_matrix((n, n))
+        for i in range(n):
+            near = np.setdiff1d(np.arange(max(0, i - reach), min(n, i + reach)), [i])
+            take = (width - 1) // 2 if i % 5 == 0 else width - 1
+            for j in rng.choice(near, take, replace=False):
+                A[i, j] = rng.uniform(-1.0, 0.3)
+        A = A.tocsr()
+        A = (A + sp.diags(1.2 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)).tocsr()
+        A.sort_indices()
+        x = rng.standard_normal(n)
+        M = P.Matrix(hip, A.indptr, A.indices, A.data)
+        y = P.solver.BiCGSTAB(tol=bound, precision=precision).step(M, np.zeros(n), A @ x)
+        # x - y = A^-1 r, ||A^-1||_inf <= 1 / min(diagonal - off-diagonals) <= 1 / 0.1, ||r||_inf <= ||r||_2
+        assert np.abs(y - x).max() <= 10.0 * bound * np.linalg.norm(A @ x) + 1e-13 * np.abs(x).max()
