@@ -172,6 +172,11 @@ template <typename T>
 constexpr int keptRows() { return sizeof(T) == 8 ? 3 : 4; }
 template <typename T>
 constexpr int heldRows() { return sizeof(T) == 8 ? 4 : 6; }
+// Rows per thread at most (see resident_plan).
+template <typename T>
+constexpr int mostRows(bool dia, int W) {
+    return W == 16 ? 1 : dia && W <= 7 ? (sizeof(T) == 4 ? 6 : 5) : keptRows<T>();
+}
 
 // FP64: plain row products; FP32: the difference form (matRow in krylov.hip; the diagonal
 // coefficient holds the row sum, or zero where the matrix has zero row sums).
@@ -570,23 +575,12 @@ void launchOne(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv) {
                  rv.blocks + (rv.blocks > 1 ? 1 : 0), BS, kv, rv);
 }
 
-template <typename T, bool DIA, int W>
-void launchR(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, int R) {
-    switch (R) {
-    case 1: launchOne<T, DIA, W, 1>(L, kv, rv); return;
-    case 2: launchOne<T, DIA, W, 2>(L, kv, rv); return;
-    case 3: launchOne<T, DIA, W, 3>(L, kv, rv); return;
-    case 4:
-        if constexpr (sizeof(T) == 4 || (DIA && W <= 7)) launchOne<T, DIA, W, 4>(L, kv, rv);
-        return;
-    case 5:
-        if constexpr (DIA && W <= 7) launchOne<T, DIA, W, 5>(L, kv, rv);
-        return;
-    case 6:
-        if constexpr (DIA && W <= 7 && sizeof(T) == 4) launchOne<T, DIA, W, 6>(L, kv, rv);
-        return;
-    default: throw Error(PRISM_ERR_RUNTIME, "resident BiCGSTAB: no kernel for this many rows per thread");
-    }
+// The instance with `rows` rows per thread: there is one for each number that a plan may ask for.
+template <typename T, bool DIA, int W, int R = 1>
+void launchRows(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, int rows) {
+    if (rows == R) launchOne<T, DIA, W, R>(L, kv, rv);
+    else if constexpr (R < mostRows<T>(DIA, W)) launchRows<T, DIA, W, R + 1>(L, kv, rv, rows);
+    else throw Error(PRISM_ERR_RUNTIME, "resident BiCGSTAB: no kernel for this many rows per thread");
 }
 
 }  // namespace
@@ -606,13 +600,12 @@ ResidentPlan resident_plan(int64_t n, bool dia, int wmax, int n_cu) {
     const int W = wmax <= 5 ? 5 : wmax <= 8 ? (dia && wmax <= 7 ? 7 : 8) : wmax <= 16 && !dia ? 16 : 0;
     const int most = std::min(n_cu - 1, RES_MAX_BLOCKS);
     if (!W || n < 1 || most < 1) return p;
-    const int rmax = W == 16 ? 1 : dia && W <= 7 ? (sizeof(T) == 4 ? 6 : 5) : keptRows<T>();
     int spb = 0;
     krylov_grid(n, &spb);
     int64_t rows = (int64_t)spb * 64;
     if (n > (int64_t)most * RES_BS) rows = ((n + most - 1) / most + 63) / 64 * 64;
     const int64_t R = (rows + RES_BS - 1) / RES_BS;
-    if (R > rmax) return p;
+    if (R > mostRows<T>(dia, W)) return p;
     p.blocks = (int)((n + rows - 1) / rows);
     p.rows = (int)rows;
     p.R = (int)R;
@@ -629,13 +622,13 @@ void launch_resident_mark(const Launch& L, T* p, size_t count, unsigned long lon
 template <typename T>
 void launch_resident(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, const ResidentPlan& plan) {
     if (kv.ndia) {
-        if (plan.W == 5) launchR<T, true, 5>(L, kv, rv, plan.R);
-        else if (plan.W == 7) launchR<T, true, 7>(L, kv, rv, plan.R);
-        else launchR<T, true, 8>(L, kv, rv, plan.R);
+        if (plan.W == 5) launchRows<T, true, 5>(L, kv, rv, plan.R);
+        else if (plan.W == 7) launchRows<T, true, 7>(L, kv, rv, plan.R);
+        else launchRows<T, true, 8>(L, kv, rv, plan.R);
     } else {
-        if (plan.W == 5) launchR<T, false, 5>(L, kv, rv, plan.R);
-        else if (plan.W == 8) launchR<T, false, 8>(L, kv, rv, plan.R);
-        else launchOne<T, false, 16, 1>(L, kv, rv);
+        if (plan.W == 5) launchRows<T, false, 5>(L, kv, rv, plan.R);
+        else if (plan.W == 8) launchRows<T, false, 8>(L, kv, rv, plan.R);
+        else launchRows<T, false, 16>(L, kv, rv, plan.R);
     }
 }
 
