@@ -27,3 +27,10 @@ def hip():
     be = P.Backend.hip(0)
     yield be
     be.close()
+
+
+@pytest.fixture(params=["resident", "single"])
+def iteration(request, monkeypatch):
+    """Both forms of a Krylov iteration: in one resident launch where the system fits (as a user has
+    it), and in launches of the single kernels (as on larger systems)."""
+    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "1" if request.param == "resident" else "0")

@@ -16,6 +16,7 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
+@pytest.mark.usefixtures("iteration")
 def test_advection_muscl_64(hip, ref):
     """The advection-diffusion workload at its own size (64^3, jittered +-0.2h, MUSCL, kappa
     1e-3, over-relaxed corrected diffusion), first outer iteration: A and b against the oracle
@@ -44,6 +45,7 @@ def test_advection_muscl_64(hip, ref):
         assert rel(x, sr["fp64"][0]) <= 1e-9, (prec, rel(x, sr["fp64"][0]))
 
 
+@pytest.mark.usefixtures("iteration")
 def test_simple_cavity_40(hip, ref):
     """The SIMPLE cavity workload (SMART, 0.7 / 0.3, automatic reference cell) at 40^3, one
     outer iteration (SMART's discrete switching parts round-off-different runs afterwards)."""
@@ -58,6 +60,7 @@ def test_simple_cavity_40(hip, ref):
     assert rel(out["hip"][1], out["ref"][1]) <= 1e-10
 
 
+@pytest.mark.usefixtures("iteration")
 def test_piso_taylor_green_16(hip, ref):
     """The PISO workload on 16^3 x 6 tetrahedra (divergence-free noise, dt at Courant 0.5),
     three steps, FP64 pressure: GPU against the oracle."""

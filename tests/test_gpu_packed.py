@@ -10,7 +10,7 @@ import pytest
 import prism_amd as P
 from prism_amd import cases
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("iteration")]
 
 
 def rel(a, b):

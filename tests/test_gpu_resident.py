@@ -96,6 +96,66 @@ def test_several_rows_per_thread(hip, monkeypatch, n, precision):
     assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
 
 
+def near(n, row, seed=3):
+    """`row` off-diagonals a row within 100 columns (16-bit sliced ELL), other ones in each row."""
+    rng = np.random.default_rng(seed)
+    rows = np.repeat(np.arange(n), row)
+    cols = np.clip(rows + rng.integers(-100, 100, n * row), 0, n - 1)
+    A = sp.coo_matrix((rng.uniform(-1.0, 0.3, n * row), (rows, cols)), shape=(n, n)).tocsr()
+    A.setdiag(0.0)
+    A.setdiag(1.1 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)
+    A.sort_indices()
+    return A
+
+
+EIGHT = (-500, -20, -3, -1, 1, 20, 500)
+SEVEN = (-4096, -64, -1, 1, 64, 4096)
+
+
+@pytest.mark.parametrize("build,n,arg,precision,precond", [
+    # sliced ELL, five and eight entries, two rows per thread up to the most
+    (scattered, 255 * 512 + 1, 4, "fp64", None), (scattered, 255 * 512 + 1, 7, "fp64", None),
+    (near, 255 * 1024 + 1, 4, "fp64", None), (near, 255 * 1024, 7, "fp64", None),
+    (scattered, 255 * 1536, 4, "fp64", None), (near, 255 * 1536, 7, "fp64", None),
+    (scattered, 255 * 512 + 1, 4, "fp32", None), (near, 255 * 512 + 1, 7, "fp32", None),
+    (near, 255 * 1536 + 1, 4, "fp32", None), (scattered, 255 * 1536 + 1, 7, "fp32", None),
+    (near, 255 * 2048, 4, "fp32", None), (near, 255 * 2048, 7, "fp32", None),
+    # eight diagonals
+    (diagonals, 255 * 512 + 1, EIGHT, "fp64", None), (diagonals, 255 * 1536, EIGHT, "fp64", None),
+    (diagonals, 255 * 1024 + 1, EIGHT, "fp32", None), (diagonals, 255 * 2048, EIGHT, "fp32", None),
+    # Jacobi, with coefficients kept and read again for each product
+    (diagonals, 262144, SEVEN, "fp64", "jacobi"), (near, 200001, 4, "fp64", "jacobi"),
+    (scattered, 200001, 7, "fp32", "jacobi"), (diagonals, 255 * 2048, SEVEN, "fp32", "jacobi"),
+    (diagonals, 255 * 2048 + 1, SEVEN, "fp64", "jacobi"), (diagonals, 255 * 3072, SEVEN, "fp32", "jacobi")])
+def test_every_plan_of_several_rows(hip, monkeypatch, build, n, arg, precision, precond):
+    print(f"case resident plan {build.__name__} {n} {arg} {precision} {precond}", flush=True)
+    A = build(n, arg)
+    x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision, precond=precond)
+    assert used
+    assert r.krylov_rel_residual <= 1e-12
+    assert np.linalg.norm(b - A @ x) <= 2e-12 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("nx,precond", [(128, None), (300, "sgs")])
+def test_more_iterations_than_two_launches(hip, monkeypatch, nx, precond):
+    """A weakly dominant system, one row per thread: the state goes from full launch to full launch."""
+    print(f"case resident launches {nx} {precond}", flush=True)
+    line = sp.diags([-1.0, 2.0, -1.0], [-1, 0, 1], shape=(nx, nx))
+    A = (sp.kron(sp.identity(nx), line) + sp.kron(line, sp.identity(nx))).tocsr()
+    A.sort_indices()
+    A.data *= np.where(A.data < 0, np.random.default_rng(12).uniform(0.98, 1.02, A.nnz), 1.0)
+    b = np.random.default_rng(9).standard_normal(nx * nx)
+    xs, rs = [], []
+    for resident in "10":
+        monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", resident)
+        out = []
+        xs.append(P.solver.BiCGSTAB(tol=1e-10, precond=precond).step(matrix(hip, A), 0.0 * b, b, out))
+        rs.append(out[0])
+    assert rs[0].krylov_iters > 256
+    assert (rs[0].krylov_iters, rs[0].restarts) == (rs[1].krylov_iters, rs[1].restarts)
+    np.testing.assert_array_equal(xs[0], xs[1])
+
+
 @pytest.mark.parametrize("n,offsets,precision", [
     (255 * 1536 + 1, (-4096, -64, -1, 1, 64, 4096), "fp64"), (255 * 2048, (-511, -1, 1, 511), "fp64"),
     (255 * 2048 + 1, (-4096, -64, -1, 1, 64, 4096), "fp64"), (255 * 2560, (-4097, -63, -1, 1, 63, 4097), "fp64"),

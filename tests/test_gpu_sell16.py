@@ -12,7 +12,7 @@ import scipy.sparse as sp
 import prism_amd as P
 from prism_amd import cases
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("iteration")]
 
 NX, NY, NZ = 76, 76, 2
 
@@ -77,11 +77,10 @@ def test_16_bit_offsets_against_oracle(hip, ref, mesh_data):
 
 @pytest.mark.parametrize("precision,bound", [("fp64", 1e-12), ("fp32", 1e-10)])
 @pytest.mark.parametrize("width", [1, 2, 3, 4, 8, 9, 10, 11, 12, 13, 17])
-def test_slice_widths(hip, monkeypatch, width, precision, bound):
-    """The single kernels' row products at every shape of their bodies: slices of one width, and of
+def test_slice_widths(hip, width, precision, bound):
+    """Row products at every shape of their bodies: slices of one width, and of
     smaller ones (every fifth row has half the entries), columns near (16 bits) and scattered."""
     print(f"case slice width {width} {precision}", flush=True)
-    monkeypatch.setenv("PRISM_KRYLOV_RESIDENT", "0")
     n = 1000
     for reach in (40, n):
         rng = np.random.default_rng(width)

@@ -19,6 +19,7 @@ def advection(be):
     return c
 
 
+@pytest.mark.usefixtures("iteration")
 @pytest.mark.parametrize("precision,tol,bound", [("fp64", 1e-12, 1e-10), ("fp32", 1e-10, 1e-8)])
 def test_precisions_against_oracle(hip, ref, precision, tol, bound):
     out = {}
@@ -32,6 +33,7 @@ def test_precisions_against_oracle(hip, ref, precision, tol, bound):
         assert out["hip"][1].refinements >= 2  # the FP64 residual was recomputed
 
 
+@pytest.mark.usefixtures("iteration")
 @pytest.mark.parametrize("precision,bound", [("fp64", 1e-10), ("fp32", 1e-7)])
 def test_reference_cell_system(hip, ref, precision, bound):
     """All-Neumann pressure correction with reference cell 3 and value 0.25: the device solves
@@ -48,6 +50,7 @@ def test_reference_cell_system(hip, ref, precision, bound):
     assert out["hip"][1].final_residual < 1e-8
 
 
+@pytest.mark.usefixtures("iteration")
 def test_jacobi_preconditioned(hip, ref):
     out = {}
     for name, be in (("hip", hip), ("ref", ref)):
