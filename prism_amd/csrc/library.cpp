@@ -1092,14 +1092,15 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
         rv.spin = residentSpin();
     }
     for (;;) {
-        const long long todo = std::min<long long>(resident ? quota : chunk, maxit - (k - base));
+        // the launches of the single kernels give the same bits: no waiting for a turn
+        const bool here = resident && ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu, false);
+        const long long todo = std::min<long long>(here ? quota : chunk, maxit - (k - base));
         if (todo <= 0) {
             out.done = 2;
             out.iters = k - base;
             break;
         }
-        if (resident) {
-            ticket.take(ctx->device, rv.blocks + 1, ctx->n_cu);
+        if (here) {
             rv.quota = (int)todo;
             launch_sgs_resident(L, V, rv, P.wmax, k, fresh);
             launched = seconds();
@@ -1120,7 +1121,7 @@ StepOut sgsStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* b, 
             fresh = 1;
             continue;
         }
-        if (resident) ctx->rest.endedWell();
+        if (here) ctx->rest.endedWell();
         if (s.done) {
             out.done = s.done;
             out.iters = s.k_event - base;
@@ -1467,8 +1468,9 @@ StepOut krylovStep(prism_ctx* ctx, Workspace& w, const MatRef& A, const double* 
             }
             last_iter = s.nit;
             last_rr = s.rr;
-            if (plan.blocks > 0) {
-                ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu);
+            // the single kernels sum in the same order with one row per thread (and unpacked rows)
+            const bool wait = plan.R > 1 || kv.pack;
+            if (plan.blocks > 0 && ticket.take(ctx->device, plan.blocks + 1, ctx->n_cu, wait)) {
                 launch_resident<T>(L, kv, rv, plan);
                 launched = seconds();
                 resident_last = true;

@@ -1,6 +1,6 @@
 // Which resident kernels may be in flight together (prism_amd/csrc/resident_ticket.h): the blocks of
 // every set that is let in, dealt to the XCDs in turn from any one on, fit their compute
-// units; the others wait, and are served in the order of asking.
+// units; the others wait, and are served in the order of asking, or are told that they do not fit.
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -36,26 +36,28 @@ int main() {
         // 132 and 124 blocks want 17 + 16 of 32 units: the second waits, and what asks after it
         // (small enough to go at once) does not pass it
         ResidentTicket first;
-        first.take(0, 132, cu);
+        check(first.take(0, 132, cu, false), "a kernel alone is refused", 132, 0);
         std::atomic<int> order{0};
         int big = 0, small = 0, elsewhere = 0;
         std::thread t([&] {
             ResidentTicket s;
-            s.take(0, 124, cu);
+            s.take(0, 124, cu, true);
             big = ++order;
             settle();
         });
         settle();
         std::thread u([&] {
             ResidentTicket s;
-            s.take(0, 8, cu);
+            s.take(0, 8, cu, true);
             small = ++order;
         });
         settle();
         check(order == 0, "let in beside 132 blocks", 132, 124);
+        ResidentTicket other;
+        check(!other.take(0, 8, cu, false), "passed those who wait", 8, 0);
         std::thread v([&] {
             ResidentTicket s;
-            s.take(1, cu, cu);
+            s.take(1, cu, cu, true);
             elsewhere = 1;
         });
         v.join();
@@ -64,8 +66,8 @@ int main() {
         t.join();
         u.join();
         check(big == 1 && small == 2, "order of asking", big, small);
-        first.take(0, cu, cu);
-        first.take(0, cu, cu);  // taken again: its first units are given back
+        check(first.take(0, cu, cu, false) && !other.take(0, 1, cu, false), "a full device", cu, 1);
+        check(first.take(0, cu, cu, false), "taken again: its first units are given back", cu, 0);
     }
     {
         // never more than the units of an XCD at once
@@ -76,16 +78,16 @@ int main() {
                 ResidentTicket s;
                 for (int i = 0; i < 500; ++i) {
                     const int blocks = 1 + (37 * i + 91 * k) % cu, units = ResidentTicket::share(blocks);
-                    s.take(2, blocks, cu);
+                    if (!s.take(2, blocks, cu, i % 3 != 0)) continue;
                     const int h = held += units;
                     if (h > worst) worst = h;
                     held -= units;
                     s.give();
-                    ++rounds;
+                    if (i % 3) ++rounds;
                 }
             });
         for (auto& t : ts) t.join();
-        check(rounds == 3000 && worst <= cu / XCDS, "units held at once", rounds, worst);
+        check(rounds == 6 * 333 && worst <= cu / XCDS, "units held at once", rounds, worst);
     }
     {
         // waits that run out after 0.4 s each, in a process that solves without a pause

@@ -254,8 +254,8 @@ def test_without_room_for_the_exchange(hip, monkeypatch):
 
 
 def test_two_threads_share_the_device(hip, monkeypatch):
-    """Two contexts solve at once; together their blocks exceed the device, so their launches take
-    turns: the bits of a solve alone."""
+    """Two contexts solve at once; together their blocks exceed the device, so one of them takes
+    the three-kernel iteration now and then: the same bits either way."""
     print("case resident two threads", flush=True)
     monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
     A = diagonals(100000, (-2000, -50, -1, 1, 50, 2000))
@@ -280,10 +280,13 @@ def test_two_threads_share_the_device(hip, monkeypatch):
 
 @pytest.mark.parametrize("n,offsets,precision,precond", [
     (50000, (-2000, -50, -1, 1, 50, 2000), "fp64", None),      # 98 blocks each: both run
-    (150000, (-2000, -50, -1, 1, 50, 2000), "fp64", None),     # two rows per thread
-    (64 * 64 * 40, (-4096, -64, -1, 1, 64, 4096), "fp32", None),  # the single kernels are the packed ones
+    (100000, (-2000, -50, -1, 1, 50, 2000), "fp32", None),     # one at a time; the single kernels beside it
+    (150000, (-2000, -50, -1, 1, 50, 2000), "fp64", None),     # two rows per thread: they take turns
+    (64 * 64 * 40, (-4096, -64, -1, 1, 64, 4096), "fp32", None),
     (100000, (-50, -1, 1, 50), "fp64", "sgs")])
 def test_threads_do_not_change_the_bits(hip, monkeypatch, n, offsets, precision, precond):
+    """Three contexts solve at once, beside each other, in turns, or with the single kernels where
+    these give the same bits: the bits of a solve alone."""
     print(f"case resident threads {n} {precision} {precond}", flush=True)
     monkeypatch.delenv("PRISM_KRYLOV_RESIDENT", raising=False)
     A = diagonals(n, offsets)
