@@ -130,16 +130,19 @@ template <int W>
 __global__ void __launch_bounds__(BS) k_sgs_resident(SgsView V, SgsResidentView R, long long k0, int fresh) {
     constexpr unsigned long long MARK = Word<double>::MARK;
     __shared__ double sh[2 * NW + 2], sh0[3 * SUBW];
-    __shared__ int fail;
+    __shared__ int fail, gone;
     SgsState* st = V.st;
     const int tid = threadIdx.x, lane = tid & 63, G = R.blocks, n = V.n, nc = V.nc;
     const int lb = (int)blockIdx.x < G ? (int)blockIdx.x : G;
-    // first of all, whatever else this launch does: the next one takes these words as unwritten
+    // One thread's reading of the event words decides for its block: a launch whose first test finds an
+    // event ends without any exchange, so block 0 may write it while other blocks begin.  Those
+    // that see it leave whole, their stale words marked; the others find the same event themselves.
+    const int event = st->done | st->flag | st->stuck;
     if (tid < RES_LINE * (lb < G ? 1 : RES_COPIES)) post(&R.stale[RES_LINE * lb + tid], MARK);
-    // done and flag: the same values in every thread of the grid, as a launch writes them only after
-    // a round of totals.  stuck can be new here: then this launch's results count for nothing.
-    if (st->done | st->flag | st->stuck) return;
-    if (tid == 0) fail = 0;
+    if (tid == 0) {
+        fail = 0;
+        gone = event;
+    }
     // totals of the last X (or the seed), as the first kernel of an iteration forms them
     double red[3];
 #pragma unroll
@@ -152,6 +155,7 @@ __global__ void __launch_bounds__(BS) k_sgs_resident(SgsView V, SgsResidentView 
         if (tid < SGS_BS && lane == 0) sh0[q * SUBW + (tid >> 6)] = s;
     }
     __syncthreads();
+    if (gone) return;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         double s = 0.0;
@@ -308,13 +312,6 @@ __global__ void __launch_bounds__(BS) k_sgs_resident(SgsView V, SgsResidentView 
         markSums(LINE_X, 2 * SUB);
         rho_old = rho;
         ++m;
-    }
-    // An event of the first test, before any exchange: one round, so that every block has read the
-    // event words and marked its stale ones before block 0 writes the event.
-    if (m == 0) {
-        const double none[2] = {0.0, 0.0};
-        double all[2];
-        if (!totals<2>(S, LINE_X, none, all, own)) return;
     }
     if (m > 0 && ok) {
         V.x[i] = x;
