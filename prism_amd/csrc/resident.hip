@@ -10,8 +10,9 @@
 // one: 200 rows FP64 14 -> 2.6 us, 16,384 rows FP64 15 -> 5.8 us, 82,944 rows of tetrahedra
 // FP32 17.5 -> 7.0 us, 110,592 rows FP64 17 -> 7.8 us, 262,144 rows FP64 19.3 -> 10.0 us,
 // 512,000 rows FP64 29.8 -> 18.7 us.  What bounds it now is latency: four to five hops of
-// 0.3-0.5 us between blocks per iteration, and at two and three rows per thread the products'
-// wait for their neighbours' words (0.7 us per row and product).
+// 0.3-0.5 us between blocks per iteration, and at two and three rows per thread (262,144 rows
+// are 1,088 a block: three in one wave of eight) the products' wait for their neighbours' words
+// (0.7 us per row and product).
 //
 // Exchange without barriers.  A word that another block waits for carries its own flag: it
 // holds the mark, a signalling NaN that no arithmetic produces (results are quiet NaNs), until
@@ -34,7 +35,8 @@
 // totals two.  Elements of the block's own rows are read from LDS instead.
 //
 // The reductions sum per thread, wave, block and then over the blocks in index order, with one
-// row per thread in exactly the order of the three-kernel iteration.  One block more than
+// row per thread in exactly the order of the three-kernel iteration (of its kernels with a row per
+// thread; those with packed rows have another).  One block more than
 // the rows need does nothing else: a block that also has rows delays every reduction by its
 // own products (64^3: 12.2 us per iteration instead of 11.0).
 //
@@ -140,10 +142,11 @@ __device__ inline bool awaitTotals(unsigned long long* slot, int G, int lb, unsi
 
 // Orders the reads of a row's elements before their first use: one wait for all of them.  (Left
 // alone, the compiler reads each into the same register and waits for it, W LDS latencies in a
-// row.)  Up to two rows per thread in FP64, four in FP32: 82,944 rows of tetrahedra in FP32 go
-// from 360 to 337 us per launch, 64^3 rows in FP64 stay at 10 us per iteration (the wait for the
-// neighbours' words is longer there); with more rows it spills up to 24 more registers, and 512,000
-// rows FP64 went from 18.7 to 19.1 us per iteration.
+// row.)  Up to two rows per thread in FP64, four in FP32: per iteration, without / with, seven
+// diagonals, FP64 110,592 rows (one) 8.6 / 8.4 us, 180,000 rows (two) 8.9 / 8.6 us, FP32 262,144
+// rows (three) 10.2 / 9.3 us, 512,000 rows (four) 12.4 / 10.4 us; 82,944 rows of tetrahedra in FP32
+// 360 / 337 us per launch.  With more rows it spills up to 24 more registers, and 512,000 rows
+// FP64 went from 18.7 to 19.1 us per iteration.
 template <typename U, int W>
 __device__ inline void together(U (&l)[W]) {
     if constexpr (W == 5) {
@@ -500,8 +503,9 @@ __global__ void __launch_bounds__(BS) k_resident(KView<T> kv, ResidentView<T> rv
     }
 
     // The totals say that every block has posted its sums, not that it has read its neighbours' p_k
-    // yet: one more round (the next four sums' words are free), after which p_k can be marked, and
-    // no block can give up any more when the first one writes the state.
+    // yet: one more round (the next four sums' words are free), after which p_k can be marked.  A
+    // block whose wait for this round's totals runs out leaves its old x beside the others' new
+    // one: a valid guess, as the host starts anew from x and looks at nothing else (stuck).
     if (G > 1) {
         const double none[2] = {0.0, 0.0};
         double all[2];
@@ -592,7 +596,7 @@ void launchRows(const Launch& L, const KView<T>& kv, const ResidentView<T>& rv, 
 // many blocks as there can be, so that the rows of a block, and with them an iteration's
 // work, are fewest.  Where the line lies: with up to seven diagonals, FP64 5 rows per thread
 // (652,800 in all) 27.6 us per iteration against 31.9 us of the three kernels at 643,280 rows
-// (its 87 spilled registers leave no room for a sixth); FP32 6 rows (783,360 in all) 18.6 us against 32.8 us (row per thread) at
+// (its 84 spilled registers leave no room for a sixth); FP32 6 rows (783,360 in all) 18.6 us against 32.8 us (row per thread) at
 // 665,280, while 7 take 25.8 us against 24.9 us of the packed kernels at 847,872.  Else as many
 // as hold their coefficients in registers (keptRows), one with up to 16 entries per row.
 template <typename T>
