@@ -194,6 +194,7 @@ def test_wait_that_runs_out_falls_back(hip, monkeypatch, precision):
     """One poll per wait: the blocks give up at their first wait, and the solve goes on with the
     three-kernel iteration."""
     print(f"case resident spin {precision}", flush=True)
+    hip = P.Backend.hip(0)  # it rests from resident kernels afterwards: not the other tests' context
     monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
     A = scattered(9001, 7)
     x, b, r, used = solve(hip, A, monkeypatch, True, precision=precision)
@@ -226,7 +227,10 @@ def test_waits_that_run_out_are_remembered(hip, monkeypatch, precond, kernel):
     # a context that forgets would launch one in each solve
     assert 1 <= launches(200) < 200
     monkeypatch.delenv("PRISM_KRYLOV_SPIN")
-    time.sleep(2.0)
+    for _ in range(300):  # a rest is 1024 times the last wait's 0.1 ms or less, as a rule
+        if launches(1):
+            break
+        time.sleep(0.1)
     assert launches(5) >= 5
     be.close()
 
@@ -378,6 +382,7 @@ def test_state_handed_from_launch_to_launch(hip, monkeypatch, name, precision, p
 
 def test_sgs_wait_that_runs_out_falls_back(hip, monkeypatch):
     print("case resident sgs spin", flush=True)
+    hip = P.Backend.hip(0)
     monkeypatch.setenv("PRISM_KRYLOV_SPIN", "1")
     A = diagonals(5000, (-22, -1, 1, 22))
     x, b, r, _ = solve(hip, A, monkeypatch, True, precond="sgs")
